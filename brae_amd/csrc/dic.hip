@@ -11,6 +11,7 @@
 // with its own level schedule (device_sym_gauss_seidel.cuh, device_dilu.cuh).
 #include "amg.hpp"
 #include "reduce.hpp"
+#include "sweep.hpp"
 
 #include <algorithm>
 
@@ -251,6 +252,7 @@ __global__ void dicResK(double* st, int* fl)
 
 void dicApply(Ctx& c, Mesh& m, const LduView& A, const double* rD, const double* r, double* w, const int* stop)
 {
+    if (sweepSubstitute(c, m, rD, A.upper, A.upper, r, w, stop)) return;
     const LevelSched& s = *m.sched;
     for (size_t l = 0; l + 1 < s.fwdStart.size(); ++l)
     {
@@ -268,6 +270,7 @@ void dicApply(Ctx& c, Mesh& m, const LduView& A, const double* rD, const double*
 
 void dicFactor(Ctx& c, Mesh& m, const LduView& A, double* rD, const int* stop)
 {
+    if (sweepFactor(c, m, A.diag, A.upper, A.upper, rD)) return;
     const LevelSched& s = *m.sched;
     for (size_t l = 0; l + 1 < s.fwdStart.size(); ++l)
     {
@@ -297,6 +300,7 @@ void launchGaussSeidel(Ctx& c, Mesh& m, const LduView& A, const double* b, doubl
     if (A.lower != A.upper) throw Error(kErrUnsupported, "mfv: Gauss-Seidel here takes a symmetric matrix");
     if (!m.nCells) return;
     buildLevels(c, m);
+    if (sweepGaussSeidel(c, m, A.diag, A.upper, b, psi, nSweeps, bPrime)) return;
     const LevelSched& s = *m.sched;
     for (int sw = 0; sw < nSweeps; ++sw)
     {

@@ -166,6 +166,13 @@ struct LevelSched
     DBuf<int> fwdCells, bwdCells;          // [nCells] each
 };
 
+// the level schedule laid out for the one-launch sweeps (sweep.hip)
+struct SweepPlan;
+struct SweepPlanDeleter
+{
+    void operator()(SweepPlan* p) const;
+};
+
 // PBiCGStab's work vectors, kept on the mesh between solves (pbicgstab.hip)
 struct BicgWork;
 struct BicgWorkDeleter
@@ -191,6 +198,7 @@ struct Mesh
     int band = 0;              // largest neighbour - owner over the internal faces
     std::vector<label> hOwner, hNeighbour, hBFaceCell;
     std::unique_ptr<LevelSched> sched;   // built on first use by the sequential sweeps (DIC, Gauss-Seidel)
+    std::unique_ptr<SweepPlan, SweepPlanDeleter> sweep;   // on first use by a sweep on the schedule
     std::unique_ptr<BicgWork, BicgWorkDeleter> bicg;   // PBiCGStab's vectors, on first use
 };
 

@@ -16,6 +16,7 @@
 // the flag every checkEvery iterations.
 #include "amg.hpp"
 #include "reduce.hpp"
+#include "sweep.hpp"
 
 #include <mutex>
 
@@ -485,6 +486,7 @@ struct BicgRun
             diagApplyK<<<blocks(n), kTpb, 0, c.stream>>>(n, w.rD, r, y, w.fl);
             return;
         }
+        if (sweepSubstitute(c, m, w.rD, A.upper, A.lower, r, y, w.fl + BF_STOP)) return;
         const LevelSched& s = *m.sched;
         for (size_t l = 0; l + 1 < s.fwdStart.size(); ++l)
         {
@@ -506,6 +508,7 @@ struct BicgRun
             diagInvK<<<blocks(n), kTpb, 0, c.stream>>>(n, w.diagC, w.rD);
             return;
         }
+        if (sweepFactor(c, m, w.diagC, A.upper, A.lower, w.rD)) return;
         const LevelSched& s = *m.sched;
         for (size_t l = 0; l + 1 < s.fwdStart.size(); ++l)
         {

@@ -1,0 +1,1020 @@
+// The sequential sweeps of OpenFOAM's preconditioners and smoothers, one launch per sweep.
+//
+// A sweep in index order is a chain of dependencies, as deep as the mesh's level schedule: on 64^3 cells 190
+// levels of 1,400 cells, on a 2-D mesh of 12,000 cells 250 levels of 50. What bounds it is the time from one
+// level to the next, not bytes or arithmetic. A launch per level costs 3 us of kernel (four dependent loads:
+// cell, run, face and neighbour, value) and about 1 us between kernels. Here:
+//   - the addressing is laid out once per mesh in level order (SweepPlan), so that the address of everything
+//     but the neighbours' values follows from a cell's place in the order and is loaded steps ahead;
+//   - up to kLdsCells cells, one workgroup walks every level with the swept values in its LDS and a
+//     workgroup barrier between levels; a small launch before it gathers the coefficients into the order
+//     the walk reads them in (one CU's gathers would cost more than the chain);
+//   - above that, waves take chunks of one level in order and hand values on through memory, each value
+//     tagged so that a reader knows it without any fence or barrier (flow* below).
+// Each cell's arithmetic is the host loop's, in its face order, so the results are the launch-per-level
+// path's and the host's to the bit.
+// Measured, a launch per level before: one DILU application on 64^3 cells (forward and backward, 380 levels)
+// 1,280 -> 196 us, 0.5 us a level, the time a value takes between two CUs; OpenFOAM's GAMG with Gauss-Seidel
+// on a 2-D mesh of 12,180 cells 470 -> 70 ms.
+#include "sweep.hpp"
+
+#include <algorithm>
+
+namespace mfv {
+
+// Plan of one mesh's sweeps. "Place" is a cell's index in the forward level order; values in LDS and in the
+// hand-over buffer are kept by place, so a level's reads and writes are mostly contiguous. A step is a run
+// of at most `threads` cells of one level. Entry k of its lane i -- a face (-1: none), and where its
+// neighbour's value is -- is entry first + k*cells + i; in an LDS plan, whose values are found at byte
+// offsets, a lane's entries lie in pairs, for loads of two.
+struct Walk
+{
+    int nSteps = 0, nEntries = 0;
+    DBuf<int4> steps;         // {first lane, cells, first entry, entries per cell}
+    DBuf<int> cell, self;     // per lane: the cell; its place, or (Gauss-Seidel) its number of lower faces
+    DBuf<int> face, pos;      // entries
+    DBuf<int> entryCell;      // LDS: the entry's cell
+    DBuf<unsigned> at;        // LDS: in place of pos
+};
+
+struct SweepPlan
+{
+    bool usable = false;      // false: the mesh keeps a launch per level
+    bool lds = false;
+    bool wide = false;        // a cell with more lower or owned faces than the narrow kernels load ahead
+    bool packed = false;      // LDS: the substitution's coefficients are the last factorisation's
+    int n = 0, threads = 64;
+    const Ctx* owner = nullptr;   // the buffers below belong to one context's stream
+    Walk fwd, bwd;            // lower faces ascending; owned faces descending
+    bool gsReady = false, gsUsable = false;
+    Walk gs;                  // Gauss-Seidel's forward walk: both runs of faces, ascending
+    int gsAhead = 0;          // its entries loaded ahead
+    // LDS: coefficients and cell values in the walks' orders
+    DBuf<double> aFwd, aBwd, dFwd, aGs, aGsBack, gsIn;
+    // flow: the hand-over buffer and {next chunk, waves done, tag}
+    DBuf<unsigned long long> hand;
+    DBuf<unsigned> state;
+};
+void SweepPlanDeleter::operator()(SweepPlan* p) const { delete p; }
+
+namespace {
+
+// 160,008 of the 163,840 bytes of LDS a workgroup may hold. At the line the LDS walk is the faster: a DILU
+// solve takes 1.4 ms on 18,850 cells (77 levels, 0.35 us a level), 2.1 ms on 32^3 by flow (94 levels).
+constexpr int kLdsCells = 20000;
+constexpr int kLdsThreads = 512;
+// Above this a mesh keeps a launch per level: the gain falls as the levels widen and the values' words (16
+// bytes) become traffic. A DILU solve of n^3 cells against a launch per level: 6.6x at 64^3, 6.0x at 128^3,
+// 3.3x at 200^3, 2.0x at 272^3 (20 M cells, 165 -> 83 ms); the plan takes about 90 bytes a cell.
+constexpr int kFlowMaxCells = 1 << 25;
+// Entries of a step's cell that are loaded ahead, by the most that a cell of the mesh has (a hex mesh's have
+// three lower and three owned faces, agglomerated ones more); a cell's entries past these are loaded where
+// they are used. Substitution in LDS (in pairs) and by flow, Gauss-Seidel in LDS and by flow:
+constexpr int kLdsNarrow = 4, kFlowNarrow = 3, kWide = 8;
+constexpr int kGsNarrow = 6, kGsMiddle = 8, kGsWide = 12;
+
+// LDS-only ordering between a step's writes and the next one's reads: a full __syncthreads would also wait
+// for the loads in flight for later steps.
+__device__ __forceinline__ void ldsBarrier()
+{
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
+// ---------------- one workgroup, the values in LDS ----------------
+
+struct LdsWalk
+{
+    int nSteps;
+    const int4* __restrict__ steps;
+    const int* __restrict__ cell;
+    const int* __restrict__ self;
+    const unsigned* __restrict__ at;   // the entries' values: byte offsets in LDS
+    const double* __restrict__ a;      // the entries' coefficients
+};
+
+// A lane's step as loaded ahead: its first W entries (a step holds at least W per cell), two values of the
+// cell (v, d0), and where its own value is. One wave's instructions, at four cycles each, are most of a
+// step, so: addresses are a uniform base and the lane's offset, and an absent entry needs no test -- its
+// coefficient is 0 and its value a 1 kept after the last cell's, and s - 0*1 and s - 0/1 are s.
+template <int W>
+struct Step
+{
+    int first, cnt, w, e;   // uniform
+    unsigned at[W];
+    double a[W], v, d0;
+    int c;
+    unsigned own;
+};
+
+__device__ __forceinline__ double& ldsAt(double* val, unsigned byteOffset)
+{
+    return *reinterpret_cast<double*>(reinterpret_cast<char*>(val) + byteOffset);
+}
+
+// Lanes past the step's cells and steps past the walk's end read the last ones: every load is unconditional
+// and in bounds, so they issue together and none waits behind a branch. i: the lane's cell in the step.
+template <int W>
+__device__ __forceinline__ unsigned stepLoad(const LdsWalk& P, const int4 d, Step<W>& q)
+{
+    q.first = d.x;
+    q.cnt = d.y;
+    q.e = d.z;
+    q.w = d.w;
+    const unsigned i = (unsigned)min((int)threadIdx.x, d.y - 1);
+#pragma unroll
+    for (int k = 0; k < W; k += 2)
+    {
+        const uint2* at = reinterpret_cast<const uint2*>(P.at + (d.z + k * d.y));
+        const double2* a = reinterpret_cast<const double2*>(P.a + (d.z + k * d.y));
+        const uint2 p = at[i];
+        const double2 c = a[i];
+        q.at[k] = p.x;
+        q.at[k + 1] = p.y;
+        q.a[k] = c.x;
+        q.a[k + 1] = c.y;
+    }
+    return i;
+}
+
+// A walk with A step buffers that take turns (nothing in flight is copied, a copy would wait for it): while
+// step s is computed, step s + A - 1 is loaded, with what the walk adds to it (more(step, i): loads at
+// addresses that follow from the descriptor), and for step s + 2 what is found through a loaded index
+// (gather). The step's own values are read from LDS first; compute(step, values) is the rest.
+template <int W, int A, typename More, typename Gather, typename Compute>
+__device__ __forceinline__ void ldsWalk(const LdsWalk& P, double* val, More more, Gather gather, Compute compute)
+{
+    const int n = P.nSteps;
+    Step<W> q[A];
+    int4 d[A];
+#pragma unroll
+    for (int u = 0; u < A; ++u) d[u] = P.steps[min(u, n - 1)];
+#pragma unroll
+    for (int u = 0; u < A - 1; ++u)
+    {
+        more(q[u], stepLoad<W>(P, d[u], q[u]));
+        d[u] = P.steps[min(u + A, n - 1)];
+    }
+    gather(q[0]);
+    gather(q[1]);
+    for (int s = 0; s < n; s += A)
+    {
+#pragma unroll
+        for (int u = 0; u < A; ++u)
+        {
+            if (s + u >= n) break;
+            constexpr int last = A - 1;
+            const int v = (u + last) % A;
+            double x[W];
+#pragma unroll
+            for (int k = 0; k < W; ++k) x[k] = ldsAt(val, q[u].at[k]);
+            more(q[v], stepLoad<W>(P, d[v], q[v]));
+            d[v] = P.steps[min(s + u + last + A, n - 1)];
+            gather(q[(u + 2) % A]);
+            compute(q[u], x);
+            ldsBarrier();
+        }
+    }
+}
+// buffers of a walk without and with gathers
+constexpr int kAhead = 4, kAheadGather = 6;
+
+// v after the entries of a lane's step: fn(v, coefficient, value, entry) per entry in order (Down: from the
+// last). Entries past the W loaded ahead are read where they are used.
+template <int W, bool Down, typename Fn>
+__device__ __forceinline__ double entries(const LdsWalk& P, const Step<W>& q, double* val, const double (&x)[W],
+                                          double v, Fn fn)
+{
+    auto far = [&](int k) {
+        const unsigned e = q.e + (k & ~1) * q.cnt + 2 * threadIdx.x + (k & 1);
+        v = fn(v, P.a[e], ldsAt(val, P.at[e]), k);
+    };
+    const bool on = (int)threadIdx.x < q.cnt;
+    if (Down && q.w > W && on)
+        for (int k = q.w - 1; k >= W; --k) far(k);
+#pragma unroll
+    for (int j = 0; j < W; ++j)
+    {
+        const int k = Down ? W - 1 - j : j;
+        v = fn(v, q.a[k], x[k], k);
+    }
+    if (!Down && q.w > W && on)
+        for (int k = W; k < q.w; ++k) far(k);
+    return v;
+}
+
+// d = diag - sum upper*lower/d[lower neighbour]; P.a holds upper*lower, dFwd the diagonal in and 1/d out
+template <int W>
+__global__ __launch_bounds__(kLdsThreads) void ldsFactorK(int n, LdsWalk P, double* dFwd, double* __restrict__ rD)
+{
+    extern __shared__ double val[];
+    if (threadIdx.x == 0) val[n] = 1.0;
+    ldsBarrier();
+    ldsWalk<W, kAhead>(
+        P, val,
+        [&](Step<W>& q, unsigned i) {
+            const double* dg = dFwd + q.first;
+            const int* cell = P.cell + q.first;
+            q.v = dg[i];
+            q.c = cell[i];
+        },
+        [](Step<W>&) {},
+        [&](const Step<W>& q, const double (&x)[W]) {
+            const double v = entries<W, false>(P, q, val, x, q.v, [](double s, double a, double y, int) { return s - a / y; });
+            if ((int)threadIdx.x >= q.cnt) return;
+            val[q.first + threadIdx.x] = v;
+            const double inv = 1.0 / v;
+            rD[q.c] = inv;
+            dFwd[q.first + threadIdx.x] = inv;
+        });
+}
+
+// y = rD*r, y -= (rD*lower)*y forward, y -= (rD*upper)*y backward; the products are in the walks' a
+template <int W>
+__global__ __launch_bounds__(kLdsThreads) void ldsSubstK(int n, LdsWalk F, LdsWalk B, const double* __restrict__ dFwd,
+                                                         const double* __restrict__ r, double* __restrict__ y,
+                                                         const int* __restrict__ stop)
+{
+    extern __shared__ double val[];
+    if (stop && *stop) return;
+    if (threadIdx.x == 0) val[n] = 1.0;
+    ldsBarrier();
+    auto sub = [](double s, double a, double x, int) { return s - a * x; };
+    ldsWalk<W, kAheadGather>(
+        F, val,
+        [&](Step<W>& q, unsigned i) {
+            const double* rd = dFwd + q.first;
+            const int* cell = F.cell + q.first;
+            q.d0 = rd[i];
+            q.c = cell[i];
+        },
+        [&](Step<W>& q) { q.v = r[q.c]; },
+        [&](const Step<W>& q, const double (&x)[W]) {
+            const double v = entries<W, false>(F, q, val, x, q.d0 * q.v, sub);
+            if ((int)threadIdx.x < q.cnt) val[q.first + threadIdx.x] = v;
+        });
+    ldsWalk<W, kAhead>(
+        B, val,
+        [&](Step<W>& q, unsigned i) {
+            const int* cell = B.cell + q.first;
+            const int* self = B.self + q.first;
+            q.c = cell[i];
+            q.own = 8u * (unsigned)self[i];
+        },
+        [](Step<W>&) {},
+        [&](const Step<W>& q, const double (&x)[W]) {
+            const double v = entries<W, false>(B, q, val, x, ldsAt(val, q.own), sub);
+            if ((int)threadIdx.x >= q.cnt) return;
+            ldsAt(val, q.own) = v;
+            y[q.c] = v;
+        });
+}
+
+// Gauss-Seidel: psi in LDS; a cell reads its lower neighbours' new values and its upper neighbours' old ones,
+// as the in-place host loop does. in: b, the diagonal and psi by place, then room for bPrime.
+template <int W, int WB, bool Sym>
+__global__ __launch_bounds__(kLdsThreads) void ldsGsK(int n, LdsWalk F, LdsWalk B, double* in, double* __restrict__ psi,
+                                                      int nSweeps)
+{
+    extern __shared__ double val[];
+    const int tid = threadIdx.x;
+    double* bPrime = in + 3 * (size_t)n;
+    for (int i = tid; i < n; i += blockDim.x) val[i] = in[2 * (size_t)n + i];
+    if (tid == 0) val[n] = 1.0;
+    __syncthreads();
+    for (int sw = 0; sw < nSweeps; ++sw)
+    {
+        ldsWalk<W, kAhead>(
+            F, val,
+            [&](Step<W>& q, unsigned i) {
+                const double* b = in + q.first;
+                const double* dg = in + n + q.first;
+                q.v = b[i];
+                q.d0 = dg[i];
+                if (Sym)
+                {
+                    const int* low = F.self + q.first;
+                    q.c = low[i];
+                }
+            },
+            [](Step<W>&) {},
+            [&](const Step<W>& q, const double (&x)[W]) {
+                double low = q.v;   // b less the lower neighbours' terms
+                const double t = entries<W, false>(F, q, val, x, q.v, [&](double s, double a, double y, int k) {
+                    const double v = s - a * y;
+                    if (Sym) low = k + 1 == q.c ? v : low;
+                    return v;
+                });
+                const double v = t / q.d0;
+                if (tid >= q.cnt) return;
+                if (Sym) bPrime[q.first + tid] = low;
+                val[q.first + tid] = v;
+            });
+        if (!Sym) continue;
+        __syncthreads();   // bPrime, written by the forward walk's lanes, is read by the reverse walk's
+        // the reverse walk: the backward entries from the last (owned faces ascending)
+        ldsWalk<WB, kAheadGather>(
+            B, val,
+            [&](Step<WB>& q, unsigned i) {
+                const int* self = B.self + q.first;
+                q.c = self[i];
+            },
+            [&](Step<WB>& q) {
+                q.v = bPrime[q.c];
+                q.d0 = in[n + q.c];
+            },
+            [&](const Step<WB>& q, const double (&x)[WB]) {
+                const double t = entries<WB, true>(B, q, val, x, q.v,
+                                                   [](double s, double a, double y, int) { return s - a * y; });
+                const double v = t / q.d0;
+                if (tid < q.cnt) val[q.c] = v;
+            });
+        __syncthreads();
+    }
+    __syncthreads();
+    for (int i = tid; i < n; i += blockDim.x) psi[F.cell[i]] = val[i];
+}
+
+// coefficients and cell values into the walks' orders
+constexpr int kTpb = 256;
+
+__global__ __launch_bounds__(kTpb) void packFactorK(int nE, const int* __restrict__ face, int n,
+                                                    const int* __restrict__ cell, const double* __restrict__ diag,
+                                                    const double* __restrict__ upper, const double* __restrict__ lower,
+                                                    double* __restrict__ a, double* __restrict__ dFwd)
+{
+    const int e = blockIdx.x * kTpb + threadIdx.x;
+    if (e < n) dFwd[e] = diag[cell[e]];
+    if (e >= nE) return;
+    const int f = face[e];
+    a[e] = f >= 0 ? upper[f] * lower[f] : 0.0;
+}
+
+// rD*lower for the forward walk's entries, then rD*upper for the backward walk's
+__global__ __launch_bounds__(kTpb) void packSubstK(int nF, const int* __restrict__ faceF, const int* __restrict__ cellF,
+                                                   int nB, const int* __restrict__ faceB, const int* __restrict__ cellB,
+                                                   const double* __restrict__ rD, const double* __restrict__ upper,
+                                                   const double* __restrict__ lower, double* __restrict__ aF,
+                                                   double* __restrict__ aB)
+{
+    const int e = blockIdx.x * kTpb + threadIdx.x;
+    if (e < nF)
+    {
+        const int f = faceF[e];
+        aF[e] = f >= 0 ? rD[cellF[e]] * lower[f] : 0.0;
+    }
+    if (e < nB)
+    {
+        const int f = faceB[e];
+        aB[e] = f >= 0 ? rD[cellB[e]] * upper[f] : 0.0;
+    }
+}
+
+__global__ __launch_bounds__(kTpb) void packGsK(int nF, const int* __restrict__ faceF, int nB,
+                                                const int* __restrict__ faceB, int n, const int* __restrict__ cell,
+                                                const double* __restrict__ diag, const double* __restrict__ upper,
+                                                const double* __restrict__ b, const double* __restrict__ psi,
+                                                double* __restrict__ aF, double* __restrict__ aB, double* __restrict__ in)
+{
+    const int e = blockIdx.x * kTpb + threadIdx.x;
+    if (e < n)
+    {
+        const int c = cell[e];
+        in[e] = b[c];
+        in[n + e] = diag[c];
+        in[2 * (size_t)n + e] = psi[c];
+    }
+    if (e < nF)
+    {
+        const int f = faceF[e];
+        aF[e] = f >= 0 ? upper[f] : 0.0;
+    }
+    if (e < nB)
+    {
+        const int f = faceB[e];
+        aB[e] = f >= 0 ? upper[f] : 0.0;
+    }
+}
+
+// ---------------- waves that hand values on ----------------
+//
+// One wave per workgroup takes chunks (steps of at most 64 cells) in order from a counter and computes each
+// as soon as the values it needs are there. A value crosses as two 8-byte words, {tag, low half} and {tag,
+// high half}, each stored and loaded as one atomic word at device scope: a reader that finds this walk's
+// tag in both has the value, whatever order they arrive in, so nothing else has to be ordered. Every wait
+// ends: a chunk needs values of earlier chunks only, those were taken earlier, by waves that were running
+// and leave no chunk unfinished; the earliest unfinished chunk never waits. The tag grows with every walk
+// (kept in device memory and advanced by the last wave to leave, so a captured launch replays correctly).
+
+struct PlanView
+{
+    int nFwd, nBwd;
+    const int4* __restrict__ steps[2];
+    const int* __restrict__ cell[2];
+    const int* __restrict__ self[2];
+    const int* __restrict__ face[2];
+    const int* __restrict__ pos[2];
+};
+
+// The addressing of one lane of a chunk: its first W entries (a chunk holds at least W per cell, the missing
+// ones marked); lanes past the chunk's cells read the last one's, so every load is unconditional.
+template <int W>
+struct Lane
+{
+    int4 d;
+    int c, self;
+    int face[W], pos[W];
+};
+
+template <int W>
+__device__ __forceinline__ void laneLoad(const int4* __restrict__ steps, int s, const int* __restrict__ cell,
+                                         const int* __restrict__ self, const int* __restrict__ face,
+                                         const int* __restrict__ pos, Lane<W>& L)
+{
+    L.d = steps[s];
+    const int j = min((int)threadIdx.x, L.d.y - 1);
+    L.c = cell[L.d.x + j];
+    L.self = self[L.d.x + j];
+#pragma unroll
+    for (int k = 0; k < W; ++k)
+    {
+        L.face[k] = face[L.d.z + k * L.d.y + j];
+        L.pos[k] = pos[L.d.z + k * L.d.y + j];
+    }
+}
+
+enum : int { kNext = 0, kDone = 1, kTag = 2, kState = 3 };
+
+__device__ __forceinline__ void put(unsigned long long* hand, int p, unsigned tag, double v)
+{
+    const unsigned long long b = __double_as_longlong(v), t = (unsigned long long)tag << 32;
+    __hip_atomic_store(hand + 2 * (size_t)p, t | (b & 0xffffffffull), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __hip_atomic_store(hand + 2 * (size_t)p + 1, t | (b >> 32), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// a value's two words as read (Both), and whether they are this walk's
+struct Both
+{
+    unsigned long long a, b;
+    __device__ __forceinline__ bool is(unsigned tag) const
+    {
+        return (unsigned)(a >> 32) == tag && (unsigned)(b >> 32) == tag;
+    }
+    __device__ __forceinline__ double value() const
+    {
+        return __longlong_as_double((long long)((a & 0xffffffffull) | (b << 32)));
+    }
+};
+
+__device__ __forceinline__ Both get(const unsigned long long* hand, int p)
+{
+    const unsigned long long* q = hand + 2 * (size_t)p;
+    return Both{__hip_atomic_load(q, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT),
+                __hip_atomic_load(q + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)};
+}
+
+__device__ __forceinline__ double await(const unsigned long long* hand, int p, unsigned tag)
+{
+    Both v = get(hand, p);
+    while (!v.is(tag))
+    {
+        __builtin_amdgcn_s_sleep(1);
+        v = get(hand, p);
+    }
+    return v.value();
+}
+
+// The values of a lane's first W entries; need: a bit per entry. Each poll reads all of them unconditionally
+// (an entry that is not needed names a place in bounds), so it costs one round trip, not one per entry.
+template <int W>
+__device__ __forceinline__ void awaitAll(const unsigned long long* hand, const int (&pos)[W], unsigned need,
+                                         unsigned tag, double (&x)[W])
+{
+    while (need)
+    {
+        Both v[W];
+#pragma unroll
+        for (int k = 0; k < W; ++k) v[k] = get(hand, pos[k]);
+#pragma unroll
+        for (int k = 0; k < W; ++k)
+            if ((need >> k & 1u) && v[k].is(tag))
+            {
+                x[k] = v[k].value();
+                need &= ~(1u << k);
+            }
+    }
+}
+
+__device__ __forceinline__ int takeChunk(unsigned* state)
+{
+    unsigned t = 0;
+    if (threadIdx.x == 0) t = __hip_atomic_fetch_add(state + kNext, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    return (int)__builtin_amdgcn_readfirstlane(t);
+}
+
+// the last wave to leave resets the counter and moves the tag on for the next launch (`by` tags were used)
+__device__ __forceinline__ void leave(unsigned* state, unsigned tag, unsigned by)
+{
+    if (threadIdx.x) return;
+    if (__hip_atomic_fetch_add(state + kDone, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1 != gridDim.x) return;
+    __hip_atomic_store(state + kNext, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __hip_atomic_store(state + kDone, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __hip_atomic_store(state + kTag, tag + by, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+template <int W, bool Factor>
+__global__ __launch_bounds__(64) void flowSubstK(PlanView P, const double* __restrict__ diag,
+                                                 const double* __restrict__ upper, const double* __restrict__ lower,
+                                                 const double* __restrict__ rD, const double* __restrict__ r,
+                                                 double* __restrict__ out, unsigned long long* hand, unsigned* state,
+                                                 const int* __restrict__ stop)
+{
+    if (stop && *stop) return;
+    const unsigned tag = __hip_atomic_load(state + kTag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    const int lane = threadIdx.x, total = P.nFwd + (Factor ? 0 : P.nBwd);
+    for (int s = takeChunk(state); s < total; s = takeChunk(state))
+    {
+        const int back = s >= P.nFwd ? 1 : 0;   // uniform
+        Lane<W> L;
+        laneLoad<W>(P.steps[back], back ? s - P.nFwd : s, P.cell[back], P.self[back], P.face[back], P.pos[back], L);
+        if (lane < L.d.y)
+        {
+            const int own = L.self;
+            const double rd = Factor ? 0.0 : rD[L.c];
+            const double v0 = back ? 0.0 : (Factor ? diag[L.c] : r[L.c]);
+            double a[W], x[W];
+            unsigned need = 0;
+#pragma unroll
+            for (int k = 0; k < W; ++k)
+            {
+                const int f = max(L.face[k], 0);
+                a[k] = Factor ? upper[f] * lower[f] : rd * (back ? upper[f] : lower[f]);
+                need |= (L.face[k] >= 0 ? 1u : 0u) << k;
+            }
+            const unsigned want = back ? tag + 1 : tag;
+            const unsigned has = need;
+            double v = back ? await(hand, own, tag) : (Factor ? v0 : rd * v0);   // there long before the neighbours'
+            awaitAll<W>(hand, L.pos, need, want, x);
+#pragma unroll
+            for (int k = 0; k < W; ++k)
+                if (has >> k & 1u) v = Factor ? v - a[k] / x[k] : v - a[k] * x[k];
+            for (int k = W; k < L.d.w; ++k)
+            {
+                const int e = L.d.z + k * L.d.y + lane, f = P.face[back][e];
+                if (f < 0) break;
+                const double xk = await(hand, P.pos[back][e], want);
+                if (Factor)
+                    v -= upper[f] * lower[f] / xk;
+                else
+                    v -= rd * (back ? upper[f] : lower[f]) * xk;
+            }
+            put(hand, own, want, v);
+            if (Factor)
+                out[L.c] = 1.0 / v;
+            else if (back)
+                out[L.c] = v;
+        }
+    }
+    leave(state, tag, 2);
+}
+
+// One Gauss-Seidel walk: forward (lower neighbours handed over; upper ones read from psi, where their old
+// values stay until this cell's is published, since their walk waits for it), or symGaussSeidel's reverse.
+template <int W, bool Back>
+__global__ __launch_bounds__(64) void flowGsK(int nSteps, const int4* __restrict__ steps, const int* __restrict__ cell,
+                                              const int* __restrict__ self, const int* __restrict__ face,
+                                              const int* __restrict__ pos, const double* __restrict__ diag,
+                                              const double* __restrict__ upper, const double* __restrict__ b,
+                                              double* psi, double* bPrime, unsigned long long* hand, unsigned* state)
+{
+    const unsigned tag = __hip_atomic_load(state + kTag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    const int lane = threadIdx.x;
+    for (int t = takeChunk(state); t < nSteps; t = takeChunk(state))
+    {
+        Lane<W> L;
+        laneLoad<W>(steps, t, cell, self, face, pos, L);
+        if (lane < L.d.y)
+        {
+            const int own = Back ? L.self : L.d.x + lane;
+            const int nl = Back ? L.d.w : L.self;   // the entries handed over: all, or the lower ones
+            double v = Back ? bPrime[L.c] : b[L.c];
+            const double dg = diag[L.c];
+            double a[W], x[W];
+            unsigned has = 0, need = 0;
+#pragma unroll
+            for (int k = 0; k < W; ++k)
+            {
+                a[k] = upper[max(L.face[k], 0)];
+                const bool on = L.face[k] >= 0;
+                has |= (on ? 1u : 0u) << k;
+                need |= (on && k < nl ? 1u : 0u) << k;
+                if (on && k >= nl) x[k] = psi[L.pos[k]];
+            }
+            awaitAll<W>(hand, L.pos, need, tag, x);
+            if (Back)
+            {
+                for (int k = L.d.w - 1; k >= W; --k)
+                {
+                    const int e = L.d.z + k * L.d.y + lane, f = face[e];
+                    if (f >= 0) v -= upper[f] * await(hand, pos[e], tag);
+                }
+#pragma unroll
+                for (int k = W - 1; k >= 0; --k)
+                    if (has >> k & 1u) v -= a[k] * x[k];
+            }
+            else
+            {
+                if (bPrime && nl == 0) bPrime[L.c] = v;
+#pragma unroll
+                for (int k = 0; k < W; ++k)
+                    if (has >> k & 1u)
+                    {
+                        v -= a[k] * x[k];
+                        if (bPrime && k + 1 == nl) bPrime[L.c] = v;
+                    }
+                for (int k = W; k < L.d.w; ++k)
+                {
+                    const int e = L.d.z + k * L.d.y + lane, f = face[e];
+                    if (f < 0) break;
+                    v -= upper[f] * (k < nl ? await(hand, pos[e], tag) : psi[pos[e]]);
+                    if (bPrime && k + 1 == nl) bPrime[L.c] = v;
+                }
+            }
+            v /= dg;
+            psi[L.c] = v;
+            put(hand, own, tag, v);
+        }
+    }
+    leave(state, tag, 1);
+}
+
+// ---------------- host ----------------
+
+bool capturing(hipStream_t s)
+{
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    return hipStreamIsCapturing(s, &st) == hipSuccess && st != hipStreamCaptureStatusNone;
+}
+
+// per cell, its faces as neighbour (ascending) and as owner (a contiguous run)
+struct Runs
+{
+    std::vector<int> ls, lo, os;
+    explicit Runs(const Mesh& m) : ls(m.nCells + 1, 0), lo(m.nFaces), os(m.nCells + 1, 0)
+    {
+        for (int f = 0; f < m.nFaces; ++f)
+        {
+            ++ls[m.hNeighbour[f] + 1];
+            ++os[m.hOwner[f] + 1];
+        }
+        for (int c = 0; c < m.nCells; ++c)
+        {
+            ls[c + 1] += ls[c];
+            os[c + 1] += os[c];
+        }
+        std::vector<int> at(ls.begin(), ls.end() - 1);
+        for (int f = 0; f < m.nFaces; ++f) lo[at[m.hNeighbour[f]]++] = f;
+    }
+};
+
+// Room for a plan's entries: a hex mesh fills about one per face and run, an agglomerated grid two or three.
+// A cell with very many faces in a wide level would pad its whole step; such a mesh keeps a launch per level.
+long long entryRoom(const Mesh& m) { return std::min(0x7fffffffLL, 16LL * ((long long)m.nCells + m.nFaces)); }
+
+// One walk: `order` cut at the levels' starts into steps of at most `threads` cells, each with room for its
+// widest cell's entries and for at least `least`. count(q): cell q's entries; list(q, put): put(face, place
+// or cell) for each in order; self(q) what the lanes carry. False where it would not fit.
+template <typename Count, typename List, typename Self>
+bool buildWalk(Ctx& c, Walk& w, const std::vector<int>& start, const std::vector<int>& order, bool lds, int threads,
+               int least, long long room, Count count, List list, Self self)
+{
+    std::vector<int4> steps;
+    long long entries = 0;
+    for (size_t l = 0; l + 1 < start.size(); ++l)
+        for (int a = start[l]; a < start[l + 1]; a += threads)
+        {
+            const int cnt = std::min(threads, start[l + 1] - a);
+            int k = least;
+            for (int i = a; i < a + cnt; ++i) k = std::max(k, count(order[i]));
+            if (lds) k = (k + 1) & ~1;
+            steps.push_back(int4{a, cnt, (int)entries, k});
+            entries += (long long)k * cnt;
+            if (entries > room) return false;
+        }
+    const size_t n = order.size();
+    std::vector<int> sf(n), face(entries, -1), pos(lds ? 0 : entries, 0), own(lds ? entries : 0, 0);
+    std::vector<unsigned> at(lds ? entries : 0, 8u * (unsigned)n);
+    for (const int4& d : steps)
+        for (int i = 0; i < d.y; ++i)
+        {
+            const int q = order[d.x + i];
+            sf[d.x + i] = self(q);
+            int k = 0;
+            list(q, [&](int f, int p) {
+                const size_t e = lds ? (size_t)d.z + (size_t)(k & ~1) * d.y + 2 * i + (k & 1)
+                                     : (size_t)d.z + (size_t)k * d.y + i;
+                ++k;
+                face[e] = f;
+                if (lds)
+                {
+                    own[e] = q;
+                    at[e] = 8u * (unsigned)p;
+                }
+                else
+                    pos[e] = p;
+            });
+        }
+    w.nSteps = (int)steps.size();
+    w.nEntries = (int)entries;
+    w.steps.upload(steps, c.stream);
+    w.cell.upload(order, c.stream);
+    w.self.upload(sf, c.stream);
+    w.face.upload(face, c.stream);
+    if (lds)
+    {
+        w.entryCell.upload(own, c.stream);
+        w.at.upload(at, c.stream);
+    }
+    else
+        w.pos.upload(pos, c.stream);
+    return true;
+}
+
+std::vector<int> placesOf(const std::vector<int>& fwd)
+{
+    std::vector<int> place(fwd.size());
+    for (size_t i = 0; i < fwd.size(); ++i) place[fwd[i]] = (int)i;
+    return place;
+}
+
+// whether the plan's arrays fit the device; without room the mesh keeps a launch per level
+template <typename Build>
+bool fits(Build build)
+{
+    try
+    {
+        return build();
+    }
+    catch (const Error& e)
+    {
+        if (e.code != kErrAlloc) throw;
+        (void)hipGetLastError();
+        return false;
+    }
+}
+
+bool planBuild(Ctx& c, Mesh& m, SweepPlan* p)
+{
+    const LevelSched& S = *m.sched;
+    const int n = m.nCells;
+    p->n = n;
+    p->owner = &c;
+    p->lds = n <= kLdsCells;
+    int widest = 1, most = 0;
+    for (const std::vector<int>* st : {&S.fwdStart, &S.bwdStart})
+        for (size_t l = 0; l + 1 < st->size(); ++l) widest = std::max(widest, (*st)[l + 1] - (*st)[l]);
+    p->threads = p->lds ? std::min(kLdsThreads, (widest + 63) / 64 * 64) : 64;
+    const std::vector<int> fwd = S.fwdCells.download(c.stream), bwd = S.bwdCells.download(c.stream);
+    const std::vector<int> place = placesOf(fwd);
+    const Runs R(m);
+    for (int q = 0; q < n; ++q) most = std::max(most, std::max(R.ls[q + 1] - R.ls[q], R.os[q + 1] - R.os[q]));
+    const int narrow = p->lds ? kLdsNarrow : kFlowNarrow;
+    p->wide = most > narrow;
+    const int least = p->wide ? kWide : narrow;
+    const auto at = [&](int q) { return place[q]; };
+    if (!buildWalk(c, p->fwd, S.fwdStart, fwd, p->lds, p->threads, least, entryRoom(m),
+                   [&](int q) { return R.ls[q + 1] - R.ls[q]; },
+                   [&](int q, auto put) {
+                       for (int k = R.ls[q]; k < R.ls[q + 1]; ++k) put(R.lo[k], place[m.hOwner[R.lo[k]]]);
+                   },
+                   at) ||
+        !buildWalk(c, p->bwd, S.bwdStart, bwd, p->lds, p->threads, least, entryRoom(m),
+                   [&](int q) { return R.os[q + 1] - R.os[q]; },
+                   [&](int q, auto put) {
+                       for (int f = R.os[q + 1] - 1; f >= R.os[q]; --f) put(f, place[m.hNeighbour[f]]);
+                   },
+                   at))
+        return false;
+    if (p->lds)
+    {
+        p->aFwd.resize(p->fwd.nEntries);
+        p->aBwd.resize(p->bwd.nEntries);
+        p->dFwd.resize(n);
+        return true;
+    }
+    p->hand.upload(std::vector<unsigned long long>(2 * (size_t)n, 0ull), c.stream);
+    p->state.upload(std::vector<unsigned>{0u, 0u, 1u}, c.stream);
+    return true;
+}
+
+// The mesh's plan, built on first use, or null: a mesh without faces or above kFlowMaxCells, a plan that
+// cannot be uploaded in a capture or would not fit, or one whose buffers another context is using.
+SweepPlan* planOf(Ctx& c, Mesh& m)
+{
+    if (!m.sched || !m.nFaces || m.nCells > kFlowMaxCells) return nullptr;
+    if (m.sweep) return m.sweep->usable && m.sweep->owner == &c ? m.sweep.get() : nullptr;
+    if (capturing(c.stream)) return nullptr;
+    std::unique_ptr<SweepPlan, SweepPlanDeleter> p(new SweepPlan());
+    if (!fits([&] { return planBuild(c, m, p.get()); })) p.reset(new SweepPlan());   // not usable
+    else p->usable = true;
+    m.sweep = std::move(p);
+    return m.sweep->usable ? m.sweep.get() : nullptr;
+}
+
+// the forward walk of Gauss-Seidel (both runs of a cell's faces); an upper neighbour's old value is found in
+// LDS by place, in memory by cell
+bool planGs(Ctx& c, Mesh& m, SweepPlan& p)
+{
+    if (p.gsReady) return p.gsUsable;
+    if (capturing(c.stream)) return false;
+    const LevelSched& S = *m.sched;
+    const std::vector<int> fwd = S.fwdCells.download(c.stream);
+    const std::vector<int> place = placesOf(fwd);
+    const Runs R(m);
+    int most = 0;
+    for (int q = 0; q < m.nCells; ++q) most = std::max(most, R.ls[q + 1] - R.ls[q] + R.os[q + 1] - R.os[q]);
+    p.gsAhead = most <= kGsNarrow ? kGsNarrow : most <= kGsMiddle ? kGsMiddle : kGsWide;
+    p.gsReady = true;
+    p.gsUsable = fits([&] {
+        if (!buildWalk(c, p.gs, S.fwdStart, fwd, p.lds, p.threads, p.gsAhead, entryRoom(m),
+                       [&](int q) { return R.ls[q + 1] - R.ls[q] + R.os[q + 1] - R.os[q]; },
+                       [&](int q, auto put) {
+                           for (int k = R.ls[q]; k < R.ls[q + 1]; ++k) put(R.lo[k], place[m.hOwner[R.lo[k]]]);
+                           for (int f = R.os[q]; f < R.os[q + 1]; ++f)
+                               put(f, p.lds ? place[m.hNeighbour[f]] : m.hNeighbour[f]);
+                       },
+                       [&](int q) { return R.ls[q + 1] - R.ls[q]; }))
+            return false;
+        if (!p.lds) return true;
+        p.aGs.resize(p.gs.nEntries);
+        p.aGsBack.resize(p.bwd.nEntries);
+        p.gsIn.resize(4 * (size_t)p.n);
+        return true;
+    });
+    return p.gsUsable;
+}
+
+PlanView flowView(const SweepPlan& p)
+{
+    return PlanView{p.fwd.nSteps, p.bwd.nSteps, {p.fwd.steps.p, p.bwd.steps.p}, {p.fwd.cell.p, p.bwd.cell.p},
+                    {p.fwd.self.p, p.bwd.self.p}, {p.fwd.face.p, p.bwd.face.p}, {p.fwd.pos.p, p.bwd.pos.p}};
+}
+
+LdsWalk ldsView(const Walk& w, const double* a)
+{
+    return LdsWalk{w.nSteps, w.steps.p, w.cell.p, w.self.p, w.at.p, a};
+}
+
+// Dynamic LDS beyond the default is opted into per kernel; a refusal leaves the launch-per-level path. The
+// call is cheap and allowed while a stream is captured.
+template <typename K>
+bool ldsAllowed(K* kernel, size_t bytes)
+{
+    if (bytes <= 65536) return true;
+    if (hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
+                            (int)bytes) == hipSuccess)
+        return true;
+    (void)hipGetLastError();
+    return false;
+}
+
+size_t ldsBytes(const SweepPlan& p) { return sizeof(double) * ((size_t)p.n + 1); }
+
+inline int blocks(int n) { return (n + kTpb - 1) / kTpb; }
+
+// waves of a flow launch, the window of chunks in work: more only poll (64^3: 256 waves 3.87 ms a solve, 1024
+// 4.21, 2048 5.22; 200^3: 34.4, 35.1, 36.6)
+constexpr int kFlowWaves = 256;
+
+template <int W>
+bool factorLds(Ctx& c, SweepPlan& p, const double* diag, const double* upper, const double* lower, double* rD)
+{
+    const size_t bytes = ldsBytes(p);
+    p.packed = ldsAllowed(&ldsFactorK<W>, bytes) && ldsAllowed(&ldsSubstK<W>, bytes);
+    if (!p.packed) return false;
+    const int nF = p.fwd.nEntries, nB = p.bwd.nEntries;
+    packFactorK<<<blocks(std::max(nF, p.n)), kTpb, 0, c.stream>>>(nF, p.fwd.face.p, p.n, p.fwd.cell.p, diag, upper, lower,
+                                                                 p.aFwd.p, p.dFwd.p);
+    ldsFactorK<W><<<1, p.threads, bytes, c.stream>>>(p.n, ldsView(p.fwd, p.aFwd.p), p.dFwd.p, rD);
+    packSubstK<<<blocks(std::max(nF, nB)), kTpb, 0, c.stream>>>(nF, p.fwd.face.p, p.fwd.entryCell.p, nB, p.bwd.face.p,
+                                                               p.bwd.entryCell.p, rD, upper, lower, p.aFwd.p, p.aBwd.p);
+    return true;
+}
+
+template <int W>
+bool substLds(Ctx& c, SweepPlan& p, const double* r, double* y, const int* stop)
+{
+    if (!p.packed) return false;
+    ldsSubstK<W><<<1, p.threads, ldsBytes(p), c.stream>>>(p.n, ldsView(p.fwd, p.aFwd.p), ldsView(p.bwd, p.aBwd.p), p.dFwd.p,
+                                                         r, y, stop);
+    return true;
+}
+
+template <int W, bool Factor>
+void substFlow(Ctx& c, SweepPlan& p, const double* diag, const double* upper, const double* lower, const double* rD,
+               const double* r, double* out, const int* stop)
+{
+    const int chunks = p.fwd.nSteps + (Factor ? 0 : p.bwd.nSteps);
+    flowSubstK<W, Factor><<<std::min(chunks, kFlowWaves), 64, 0, c.stream>>>(flowView(p), diag, upper, lower, rD, r, out,
+                                                                           p.hand.p, p.state.p, stop);
+}
+
+template <int W, int WB>
+bool gsLds(Ctx& c, SweepPlan& p, const double* diag, const double* upper, const double* b, double* psi, int nSweeps,
+           bool sym)
+{
+    const size_t bytes = ldsBytes(p);
+    if (!(sym ? ldsAllowed(&ldsGsK<W, WB, true>, bytes) : ldsAllowed(&ldsGsK<W, WB, false>, bytes))) return false;
+    const int nF = p.gs.nEntries, nB = sym ? p.bwd.nEntries : 0;
+    packGsK<<<blocks(std::max(std::max(nF, nB), p.n)), kTpb, 0, c.stream>>>(
+        nF, p.gs.face.p, nB, p.bwd.face.p, p.n, p.gs.cell.p, diag, upper, b, psi, p.aGs.p, p.aGsBack.p, p.gsIn.p);
+    const LdsWalk F = ldsView(p.gs, p.aGs.p), B = ldsView(p.bwd, p.aGsBack.p);
+    if (sym)
+        ldsGsK<W, WB, true><<<1, p.threads, bytes, c.stream>>>(p.n, F, B, p.gsIn.p, psi, nSweeps);
+    else
+        ldsGsK<W, WB, false><<<1, p.threads, bytes, c.stream>>>(p.n, F, B, p.gsIn.p, psi, nSweeps);
+    return true;
+}
+
+template <int W, bool Back>
+void gsFlow(Ctx& c, SweepPlan& p, const Walk& w, const double* diag, const double* upper, const double* b, double* psi,
+            double* bPrime)
+{
+    flowGsK<W, Back><<<std::min(w.nSteps, kFlowWaves), 64, 0, c.stream>>>(w.nSteps, w.steps.p, w.cell.p, w.self.p, w.face.p,
+                                                                        w.pos.p, diag, upper, b, psi, bPrime, p.hand.p,
+                                                                        p.state.p);
+}
+
+} // namespace
+
+bool sweepFactor(Ctx& c, Mesh& m, const double* diag, const double* upper, const double* lower, double* rD)
+{
+    SweepPlan* p = planOf(c, m);
+    if (!p) return false;
+    bool done = true;
+    if (p->lds)
+        done = p->wide ? factorLds<kWide>(c, *p, diag, upper, lower, rD) : factorLds<kLdsNarrow>(c, *p, diag, upper, lower, rD);
+    else if (p->wide)
+        substFlow<kWide, true>(c, *p, diag, upper, lower, nullptr, nullptr, rD, nullptr);
+    else
+        substFlow<kFlowNarrow, true>(c, *p, diag, upper, lower, nullptr, nullptr, rD, nullptr);
+    hipCheck(hipGetLastError(), "sweep factor");
+    return done;
+}
+
+bool sweepSubstitute(Ctx& c, Mesh& m, const double* rD, const double* upper, const double* lower, const double* r,
+                     double* y, const int* stop)
+{
+    SweepPlan* p = planOf(c, m);
+    if (!p) return false;
+    bool done = true;
+    if (p->lds)
+        done = p->wide ? substLds<kWide>(c, *p, r, y, stop) : substLds<kLdsNarrow>(c, *p, r, y, stop);
+    else if (p->wide)
+        substFlow<kWide, false>(c, *p, nullptr, upper, lower, rD, r, y, stop);
+    else
+        substFlow<kFlowNarrow, false>(c, *p, nullptr, upper, lower, rD, r, y, stop);
+    hipCheck(hipGetLastError(), "sweep substitution");
+    return done;
+}
+
+bool sweepGaussSeidel(Ctx& c, Mesh& m, const double* diag, const double* upper, const double* b, double* psi,
+                      int nSweeps, double* bPrime)
+{
+    SweepPlan* p = planOf(c, m);
+    if (!p || nSweeps <= 0 || !planGs(c, m, *p)) return false;
+    bool done = true;
+    if (p->lds)
+    {
+        const bool sym = bPrime != nullptr;
+        if (p->gsAhead == kGsNarrow)
+            done = p->wide ? gsLds<kGsNarrow, kWide>(c, *p, diag, upper, b, psi, nSweeps, sym)
+                           : gsLds<kGsNarrow, kLdsNarrow>(c, *p, diag, upper, b, psi, nSweeps, sym);
+        else if (p->gsAhead == kGsMiddle)
+            done = p->wide ? gsLds<kGsMiddle, kWide>(c, *p, diag, upper, b, psi, nSweeps, sym)
+                           : gsLds<kGsMiddle, kLdsNarrow>(c, *p, diag, upper, b, psi, nSweeps, sym);
+        else
+            done = p->wide ? gsLds<kGsWide, kWide>(c, *p, diag, upper, b, psi, nSweeps, sym)
+                           : gsLds<kGsWide, kLdsNarrow>(c, *p, diag, upper, b, psi, nSweeps, sym);
+    }
+    else
+        for (int sw = 0; sw < nSweeps; ++sw)
+        {
+            if (p->gsAhead == kGsNarrow)
+                gsFlow<kGsNarrow, false>(c, *p, p->gs, diag, upper, b, psi, bPrime);
+            else if (p->gsAhead == kGsMiddle)
+                gsFlow<kGsMiddle, false>(c, *p, p->gs, diag, upper, b, psi, bPrime);
+            else
+                gsFlow<kGsWide, false>(c, *p, p->gs, diag, upper, b, psi, bPrime);
+            if (!bPrime) continue;
+            if (p->wide)
+                gsFlow<kWide, true>(c, *p, p->bwd, diag, upper, b, psi, bPrime);
+            else
+                gsFlow<kFlowNarrow, true>(c, *p, p->bwd, diag, upper, b, psi, bPrime);
+        }
+    hipCheck(hipGetLastError(), "gauss-seidel sweep");
+    return done;
+}
+
+} // namespace mfv

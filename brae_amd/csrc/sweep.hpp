@@ -1,0 +1,24 @@
+// The sequential sweeps in one launch each (sweep.hip): DIC's and DILU's factorisation, their forward and
+// backward substitution, and Gauss-Seidel, on plans built once per mesh from its level schedule. Each
+// function returns false, having done nothing, where the sweep belongs to the caller's launch-per-level
+// path: a mesh above kFlowMaxCells, one another context sweeps, or a plan that cannot be built now. A
+// substitution goes with the last factorisation on its mesh: on small meshes that one lays the products
+// rD*lower and rD*upper out in the order the substitution reads them.
+#pragma once
+
+#include "mfv_internal.hpp"
+
+namespace mfv {
+
+// rD = 1/d, d = diag - sum over lower faces (ascending) of upper*lower/d[lower neighbour]
+bool sweepFactor(Ctx& c, Mesh& m, const double* diag, const double* upper, const double* lower, double* rD);
+// y = rD*r, forward: y -= rD*lower*y[lower neighbour] over lower faces ascending; backward:
+// y -= rD*upper*y[upper neighbour] over owned faces descending
+bool sweepSubstitute(Ctx& c, Mesh& m, const double* rD, const double* upper, const double* lower, const double* r,
+                     double* y, const int* stop);
+// nSweeps Gauss-Seidel sweeps of A psi = b (upper == lower); with bPrime each is followed by
+// symGaussSeidel's reverse walk
+bool sweepGaussSeidel(Ctx& c, Mesh& m, const double* diag, const double* upper, const double* b, double* psi,
+                      int nSweeps, double* bPrime);
+
+} // namespace mfv
