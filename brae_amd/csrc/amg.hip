@@ -1486,6 +1486,138 @@ __global__ __launch_bounds__(kTpb) void coarseInverseK(int n, int nf, const int*
     }
 }
 
+// The same inverse with [A | I] in LDS, for the coarsest grids that fit (kLdsInverse): the same element
+// updates, so the same bits. From HBM each of the n elimination steps waits for its loads several times (the
+// pivot search one row after another): 450-850 us on the 33-64 cells brae's target leaves. Here a step is three
+// barriers and a few LDS round trips, which bound it: 49 cells 102 us (454 from HBM), the largest such grids
+// 154 (850). Left of the pivot column nothing is read any more, so those
+// columns are not updated. A wave works on a row at a time; the pivot search is wave 0's while the others
+// copy the column. Rows are 2n + 1 long: a column's elements fall on different banks.
+constexpr int kLdsInverse = 96;        // 96*193*8 bytes of LDS and the face chunk, of 160 KB
+constexpr int kInvThreads = 1024;
+constexpr int kInvFaces = 512;         // faces staged at a time
+
+size_t ldsInverseBytes(int n)
+{
+    return sizeof(double) * ((size_t)n * (2 * n + 1) + n + kInvFaces) + 2 * sizeof(int) * kInvFaces;
+}
+
+__global__ __launch_bounds__(kInvThreads) void coarseInverseLdsK(int n, int nf, const int* __restrict__ own,
+                                                                 const int* __restrict__ nei,
+                                                                 const double* __restrict__ diag,
+                                                                 const double* __restrict__ upper,
+                                                                 double* __restrict__ inv)
+{
+    extern __shared__ __align__(16) uint8_t L[];
+    __shared__ double lds[kInvThreads / 64];
+    __shared__ double shScale, shPiv;
+    __shared__ int shRow;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, w = 2 * n, ld = 2 * n + 1;
+    double* M = reinterpret_cast<double*>(L);
+    double* fcol = M + (size_t)n * ld;
+    double* fu = fcol + n;
+    int* fo = reinterpret_cast<int*>(fu + kInvFaces);
+    int* fn = fo + kInvFaces;
+    for (int i = tid; i < n * ld; i += kInvThreads) M[i] = 0.0;
+    __syncthreads();
+    double dm = 0.0;
+    if (tid < n)
+    {
+        const double d = diag[tid];
+        M[tid * ld + tid] = d;
+        M[tid * ld + n + tid] = 1.0;
+        dm = fabs(d);
+    }
+    dm = blockMax<kInvThreads>(fmax(dm, 0.0), lds);
+    if (tid == 0) shScale = dm > 0.0 ? dm : 1.0;
+    // each row adds its faces in ascending order, as the sequential loop does
+    for (int f0 = 0; f0 < nf; f0 += kInvFaces)
+    {
+        const int cnt = min(kInvFaces, nf - f0);
+        __syncthreads();
+        if (tid < cnt)
+        {
+            fo[tid] = own[f0 + tid];
+            fn[tid] = nei[f0 + tid];
+            fu[tid] = upper[f0 + tid];
+        }
+        __syncthreads();
+        if (tid < n)
+            for (int f = 0; f < cnt; ++f)
+            {
+                const int o = fo[f], e = fn[f];
+                if (o == tid || e == tid) M[tid * ld + (o == tid ? e : o)] += fu[f];
+            }
+    }
+    __syncthreads();
+    for (int k = 0; k < n; ++k)
+    {
+        // the first largest |M[i][k]|, i >= k; column k as it stands
+        if (wave == 0)
+        {
+            double bv = -1.0, pv = 0.0;
+            int bi = k;
+            for (int i = k + lane; i < n; i += 64)
+            {
+                const double m = M[i * ld + k], v = fabs(m);
+                if (v > bv)
+                {
+                    bv = v;
+                    pv = m;
+                    bi = i;
+                }
+            }
+#pragma unroll
+            for (int o = 32; o > 0; o >>= 1)
+            {
+                const double ov = __shfl_xor(bv, o, 64), op = __shfl_xor(pv, o, 64);
+                const int oi = __shfl_xor(bi, o, 64);
+                if (ov > bv || (ov == bv && oi < bi))
+                {
+                    bv = ov;
+                    pv = op;
+                    bi = oi;
+                }
+            }
+            if (lane == 0)
+            {
+                // no comparable value in the column: row k stays the pivot, as in the sequential search
+                if (bv < 0.0)
+                {
+                    bi = k;
+                    pv = M[k * ld + k];
+                }
+                const double fl = 1e-14 * shScale;
+                if (!(fabs(pv) > fl)) pv = pv < 0.0 ? -fl : fl;
+                shPiv = pv;
+                shRow = bi;
+            }
+        }
+        else
+            for (int i = tid - 64; i < n; i += kInvThreads - 64) fcol[i] = M[i * ld + k];
+        __syncthreads();
+        const int p = shRow;
+        const double d = shPiv, rp = 1.0 / d;
+        // rows k and p change places; row k over the pivot
+        for (int j = k + tid; j < w; j += kInvThreads)
+        {
+            const double a = M[k * ld + j], b = M[p * ld + j];
+            M[p * ld + j] = a;
+            M[k * ld + j] = (j == k ? d : b) * rp;
+        }
+        __syncthreads();
+        for (int i = wave; i < n; i += kInvThreads / 64)
+        {
+            if (i == k) continue;
+            const double f = fcol[i == p ? k : i];
+            for (int j = k + lane; j < w; j += 64) M[i * ld + j] -= f * M[k * ld + j];
+        }
+        __syncthreads();
+    }
+    for (int i = wave; i < n; i += kInvThreads / 64)
+        for (int j = lane; j < n; j += 64) inv[i * n + j] = M[i * ld + n + j];
+}
+
 // y = A x in FP64 on the sliced rows (the fine grid's FP64 copy)
 __global__ __launch_bounds__(kTpb) void sellAmul64K(SellView S, const double* __restrict__ val,
                                                     const double* __restrict__ diag, const double* __restrict__ x,
@@ -2275,7 +2407,6 @@ void amgGalerkin(Ctx& c, Amg& a, const double* fineDiag, const double* fineUpper
                                          " cells; the dense coarsest solve takes at most " +
                                          std::to_string(kMaxDenseCoarsest));
     a.coarseInv.resize((size_t)a.nCoarsest * a.nCoarsest);
-    a.coarseWork.resize((size_t)a.nCoarsest * 2 * a.nCoarsest);
     amgCoarseMatrices(c, a, fineDiag, fineUpper);
     const int nG = (int)a.grids.size();
     // V-cycle copies of every non-coarsest grid in the working precision
@@ -2350,8 +2481,18 @@ void amgGalerkin(Ctx& c, Amg& a, const double* fineDiag, const double* fineUpper
         gl.diagV32.resize(gl.n);
         castK<float><<<blocks(gl.n), kTpb, 0, c.stream>>>(gl.n, gl.diag64.p, gl.diagV32.p);
     }
-    coarseInverseK<<<1, kTpb, 0, c.stream>>>(gl.n, gl.nFaces, gl.denseOwn.p, gl.denseNei.p, gl.diag64.p, gl.upper64.p,
-                                             a.coarseWork.p, a.coarseInv.p);
+    if (gl.n <= kLdsInverse &&
+        hipFuncSetAttribute(reinterpret_cast<const void*>(&coarseInverseLdsK), hipFuncAttributeMaxDynamicSharedMemorySize,
+                            (int)ldsInverseBytes(gl.n)) == hipSuccess)
+        coarseInverseLdsK<<<1, kInvThreads, ldsInverseBytes(gl.n), c.stream>>>(
+            gl.n, gl.nFaces, gl.denseOwn.p, gl.denseNei.p, gl.diag64.p, gl.upper64.p, a.coarseInv.p);
+    else
+    {
+        (void)hipGetLastError();
+        a.coarseWork.resize((size_t)a.nCoarsest * 2 * a.nCoarsest);
+        coarseInverseK<<<1, kTpb, 0, c.stream>>>(gl.n, gl.nFaces, gl.denseOwn.p, gl.denseNei.p, gl.diag64.p, gl.upper64.p,
+                                                 a.coarseWork.p, a.coarseInv.p);
+    }
     hipCheck(hipGetLastError(), "coarsest inverse");
     if (!a.allocatedVectors || a.vectorsFor != prec)
     {
