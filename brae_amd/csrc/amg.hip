@@ -10,6 +10,7 @@
 // reference's pivot floor 1e-14*max|diag| (device_amg_detail.cuh:93-94).
 #include "amg.hpp"
 #include "reduce.hpp"
+#include "cycle_flow.hpp"
 #include "sell_device.hpp"
 
 #include <algorithm>
@@ -48,37 +49,6 @@ __global__ __launch_bounds__(kTpb) void residualK(SellView S, const Tm* __restri
     const Tv ax = rowAx<Tm, Tv>(S, c, val, diag, scale, X);
     R.set(c, B(c) - ax);
 }
-
-// The coarse-to-fine injection, fused into whichever kernel finishes a coarse grid's cycle: coarse cell
-// C's final value goes to every fine cell of its agglomerate (the fine grid's cellStart/cellList), so
-// the fine grid reads its correction e = xc[map] as a plain vector (prolongT's values, written once).
-template <typename Tv, typename Ts>
-struct Scatter
-{
-    const int* __restrict__ start;
-    const int* __restrict__ list;
-    Ts* __restrict__ e;        // null: no fine grid waits for this one (grid 0)
-    const float* xm;           // the fine grid's multiplier
-    const int4* quads;         // the fine grid's agglomerates of up to four (may be null: the lists alone)
-    __device__ void operator()(int C, Tv v) const
-    {
-        if (!e) return;
-        const CycVec<Tv, Ts> E(e, xm);
-        if (quads)
-        {
-            const int4 q = quads[C];
-            if (q.x >= 0)
-            {
-                E.set(q.x, v);
-                if (q.y >= 0) E.set(q.y, v);
-                if (q.z >= 0) E.set(q.z, v);
-                if (q.w >= 0) E.set(q.w, v);
-                return;
-            }
-        }
-        for (int k = start[C]; k < start[C + 1]; ++k) E.set(list[k], v);
-    }
-};
 
 // xOut = x + omega*(b - A x)/D  (amgSpmvF then smoothT)
 template <typename Tm, typename Tv, typename Ts>
@@ -1916,10 +1886,18 @@ Ts* vcycleAt(Ctx& c, Amg& a, int gi, const VcycleControls& vc, const int* stop,
         coarseApplyK<Tv, Ts><<<1, kTpb, 0, c.stream>>>(n, a.coarseInv.p, v.b, v.x, v.xm, up, stop);
         return v.x;
     }
+    if (gi == a.flowStart && !c.sequentialReduce && a.coarseMode == 3)
+    {
+        ProfScope ps(c, kProfGridDown + gi);
+        if (vc.nPre == 0) zeroK<Ts><<<blocks(n), kTpb, 0, c.stream>>>(n, v.x, stop);
+        Ts* out = gi == 0 ? v.y : nullptr;   // a coarser grid's values go up through `up` alone
+        flowCycle<Tm, Tv, Ts>(c, a, vc, v.b, v.x, out, up, stop);
+        return out;
+    }
     if (gi > 0 && gi == a.tailStart && !c.sequentialReduce && a.coarseMode > 0)
     {
         ProfScope ps(c, kProfGridDown + gi);
-        if (a.coarseMode == 2 && a.tailLdsBytes > 0 && !vc.scale)
+        if (a.coarseMode >= 2 && a.tailLdsBytes > 0 && !vc.scale)
         {
             tailMixK<Tm, Tv, Ts><<<1, kTailThreads, a.tailLdsBytes, c.stream>>>(
                 reinterpret_cast<const TailGrid*>(a.tailDesc.p), reinterpret_cast<const LdsTail*>(a.tailLdsDesc.p),
@@ -2352,6 +2330,7 @@ void buildTail(Ctx& c, Amg& a)
 {
     if (a.tailFor == (int)a.prec) return;
     a.tailFor = (int)a.prec;
+    flowCycleBuild(c, a);
     const int nG = (int)a.grids.size();
     a.tailStart = 0;
     for (int g = 1; g < nG; ++g)
@@ -2577,6 +2556,10 @@ uint64_t amgLayoutKey(const Amg& a)
     auto ptr = [&mix](const void* p) { mix(reinterpret_cast<uintptr_t>(p)); };
     mix((uint64_t)a.prec);
     mix((uint64_t)a.tailStart);
+    mix((uint64_t)a.flowStart);
+    mix((uint64_t)a.coarseMode);
+    ptr(a.flowDesc.p);
+    ptr(a.flowState.p);
     mix(a.grids.size());
     for (const Grid& g : a.grids)
     {

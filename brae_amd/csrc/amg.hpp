@@ -145,12 +145,18 @@ struct Amg
     int tailStart = 0;             // first grid the single-workgroup tail kernel runs (0: none)
     DBuf<uint8_t> tailDesc;        // per tail grid: pointers and sizes for the tail kernel
     int tailFor = -1;              // precision the descriptors were built for (-1: stale)
-    int coarseMode = 2;            // 0: per-grid kernels; 1: the one-workgroup tail; 2: that tail with its
-                                   // coarsest grids staged in LDS, as many as fit (else 1)
+    int coarseMode = 3;            // 0: per-grid kernels; 1: the one-workgroup tail; 2: that tail with its
+                                   // coarsest grids staged in LDS, as many as fit (else 1); 3 (until a mode is
+                                   // set): the small grids in one launch of many waves (cycle_flow.hip)
     DBuf<uint8_t> tailLdsBlob;     // the LDS-staged tail's slice starts, 16-bit columns and lists
     DBuf<uint8_t> tailLdsDesc;     // its descriptor
     int tailLdsBytes = 0;          // LDS it needs (0: the tail does not fit; tailK runs)
     int tailLdsGrid = 0;           // the first grid staged in LDS (the tail's grids before it are read in place)
+    int flowStart = -1;            // first grid of the one-launch small grids (-1: none)
+    DBuf<uint8_t> flowDesc;        // their descriptors, columns (and the columns' coarse cells), the words values
+    DBuf<int> flowCols;            // are handed on in, and the launch's counter and tag
+    DBuf<unsigned long long> flowWords;
+    DBuf<unsigned> flowState;
     DBuf<uint8_t> cycleDesc;       // every grid's descriptor from grid 0 (batched whole solves)
     DBuf<double> batchWork;        // a batched solve's r, r_old, p, q
     bool galerkinDone = false;

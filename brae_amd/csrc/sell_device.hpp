@@ -219,5 +219,35 @@ struct CycVec<float, __half>
     __device__ void set(int i, float v) const { p[i] = __float2half(fminf(fmaxf(v * m, -65504.0f), 65504.0f)); }
 };
 
+// The coarse-to-fine injection, fused into whichever kernel finishes a coarse grid's cycle: coarse cell
+// C's final value goes to every fine cell of its agglomerate (the fine grid's cellStart/cellList), so
+// the fine grid reads its correction e = xc[map] as a plain vector (prolongT's values, written once).
+template <typename Tv, typename Ts>
+struct Scatter
+{
+    const int* __restrict__ start;
+    const int* __restrict__ list;
+    Ts* __restrict__ e;        // null: no fine grid waits for this one (grid 0)
+    const float* xm;           // the fine grid's multiplier
+    const int4* quads;         // the fine grid's agglomerates of up to four (may be null: the lists alone)
+    __device__ void operator()(int C, Tv v) const
+    {
+        if (!e) return;
+        const CycVec<Tv, Ts> E(e, xm);
+        if (quads)
+        {
+            const int4 q = quads[C];
+            if (q.x >= 0)
+            {
+                E.set(q.x, v);
+                if (q.y >= 0) E.set(q.y, v);
+                if (q.z >= 0) E.set(q.z, v);
+                if (q.w >= 0) E.set(q.w, v);
+                return;
+            }
+        }
+        for (int k = start[C]; k < start[C + 1]; ++k) E.set(list[k], v);
+    }
+};
 
 } // namespace mfv

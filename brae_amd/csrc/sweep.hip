@@ -16,6 +16,7 @@
 // Measured, a launch per level before: one DILU application on 64^3 cells (forward and backward, 380 levels)
 // 1,280 -> 196 us, 0.5 us a level, the time a value takes between two CUs; OpenFOAM's GAMG with Gauss-Seidel
 // on a 2-D mesh of 12,180 cells 470 -> 70 ms.
+#include "handover.hpp"
 #include "sweep.hpp"
 
 #include <algorithm>
@@ -52,7 +53,7 @@ struct SweepPlan
     // LDS: coefficients and cell values in the walks' orders
     DBuf<double> aFwd, aBwd, dFwd, aGs, aGsBack, gsIn;
     // flow: the hand-over buffer and {next chunk, waves done, tag}
-    DBuf<unsigned long long> hand;
+    DBuf<Word> hand;
     DBuf<unsigned> state;
 };
 void SweepPlanDeleter::operator()(SweepPlan* p) const { delete p; }
@@ -399,13 +400,9 @@ __global__ __launch_bounds__(kTpb) void packGsK(int nF, const int* __restrict__ 
 
 // ---------------- waves that hand values on ----------------
 //
-// One wave per workgroup takes chunks (steps of at most 64 cells) in order from a counter and computes each
-// as soon as the values it needs are there. A value crosses as two 8-byte words, {tag, low half} and {tag,
-// high half}, each stored and loaded as one atomic word at device scope: a reader that finds this walk's
-// tag in both has the value, whatever order they arrive in, so nothing else has to be ordered. Every wait
-// ends: a chunk needs values of earlier chunks only, those were taken earlier, by waves that were running
-// and leave no chunk unfinished; the earliest unfinished chunk never waits. The tag grows with every walk
-// (kept in device memory and advanced by the last wave to leave, so a captured launch replays correctly).
+// Workgroups of one wave take chunks (steps of at most 64 cells) in order and compute each as soon as the values
+// it needs are there, as handover.hpp describes. (Workgroups of four waves, four chunks at a time: 64^3 cells
+// 4.2 ms against 3.9, 128^3 9.8 to 18 depending on their number against 11.0.)
 
 struct PlanView
 {
@@ -444,58 +441,17 @@ __device__ __forceinline__ void laneLoad(const int4* __restrict__ steps, int s, 
     }
 }
 
-enum : int { kNext = 0, kDone = 1, kTag = 2, kState = 3 };
-
-__device__ __forceinline__ void put(unsigned long long* hand, int p, unsigned tag, double v)
-{
-    const unsigned long long b = __double_as_longlong(v), t = (unsigned long long)tag << 32;
-    __hip_atomic_store(hand + 2 * (size_t)p, t | (b & 0xffffffffull), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    __hip_atomic_store(hand + 2 * (size_t)p + 1, t | (b >> 32), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-
-// a value's two words as read (Both), and whether they are this walk's
-struct Both
-{
-    unsigned long long a, b;
-    __device__ __forceinline__ bool is(unsigned tag) const
-    {
-        return (unsigned)(a >> 32) == tag && (unsigned)(b >> 32) == tag;
-    }
-    __device__ __forceinline__ double value() const
-    {
-        return __longlong_as_double((long long)((a & 0xffffffffull) | (b << 32)));
-    }
-};
-
-__device__ __forceinline__ Both get(const unsigned long long* hand, int p)
-{
-    const unsigned long long* q = hand + 2 * (size_t)p;
-    return Both{__hip_atomic_load(q, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT),
-                __hip_atomic_load(q + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)};
-}
-
-__device__ __forceinline__ double await(const unsigned long long* hand, int p, unsigned tag)
-{
-    Both v = get(hand, p);
-    while (!v.is(tag))
-    {
-        __builtin_amdgcn_s_sleep(1);
-        v = get(hand, p);
-    }
-    return v.value();
-}
-
 // The values of a lane's first W entries; need: a bit per entry. Each poll reads all of them unconditionally
 // (an entry that is not needed names a place in bounds), so it costs one round trip, not one per entry.
 template <int W>
-__device__ __forceinline__ void awaitAll(const unsigned long long* hand, const int (&pos)[W], unsigned need,
+__device__ __forceinline__ void awaitAll(const Word* hand, const int (&pos)[W], unsigned need,
                                          unsigned tag, double (&x)[W])
 {
     while (need)
     {
-        Both v[W];
+        Hand<double>::Raw v[W];
 #pragma unroll
-        for (int k = 0; k < W; ++k) v[k] = get(hand, pos[k]);
+        for (int k = 0; k < W; ++k) v[k] = Hand<double>::get(hand, pos[k]);
 #pragma unroll
         for (int k = 0; k < W; ++k)
             if ((need >> k & 1u) && v[k].is(tag))
@@ -506,32 +462,15 @@ __device__ __forceinline__ void awaitAll(const unsigned long long* hand, const i
     }
 }
 
-__device__ __forceinline__ int takeChunk(unsigned* state)
-{
-    unsigned t = 0;
-    if (threadIdx.x == 0) t = __hip_atomic_fetch_add(state + kNext, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    return (int)__builtin_amdgcn_readfirstlane(t);
-}
-
-// the last wave to leave resets the counter and moves the tag on for the next launch (`by` tags were used)
-__device__ __forceinline__ void leave(unsigned* state, unsigned tag, unsigned by)
-{
-    if (threadIdx.x) return;
-    if (__hip_atomic_fetch_add(state + kDone, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1 != gridDim.x) return;
-    __hip_atomic_store(state + kNext, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    __hip_atomic_store(state + kDone, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    __hip_atomic_store(state + kTag, tag + by, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-
 template <int W, bool Factor>
 __global__ __launch_bounds__(64) void flowSubstK(PlanView P, const double* __restrict__ diag,
                                                  const double* __restrict__ upper, const double* __restrict__ lower,
                                                  const double* __restrict__ rD, const double* __restrict__ r,
-                                                 double* __restrict__ out, unsigned long long* hand, unsigned* state,
+                                                 double* __restrict__ out, Word* hand, unsigned* state,
                                                  const int* __restrict__ stop)
 {
     if (stop && *stop) return;
-    const unsigned tag = __hip_atomic_load(state + kTag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    const unsigned tag = launchTag(state);
     const int lane = threadIdx.x, total = P.nFwd + (Factor ? 0 : P.nBwd);
     for (int s = takeChunk(state); s < total; s = takeChunk(state))
     {
@@ -554,7 +493,7 @@ __global__ __launch_bounds__(64) void flowSubstK(PlanView P, const double* __res
             }
             const unsigned want = back ? tag + 1 : tag;
             const unsigned has = need;
-            double v = back ? await(hand, own, tag) : (Factor ? v0 : rd * v0);   // there long before the neighbours'
+            double v = back ? awaitValue<double>(hand, own, tag) : (Factor ? v0 : rd * v0);   // there long before the neighbours'
             awaitAll<W>(hand, L.pos, need, want, x);
 #pragma unroll
             for (int k = 0; k < W; ++k)
@@ -563,13 +502,13 @@ __global__ __launch_bounds__(64) void flowSubstK(PlanView P, const double* __res
             {
                 const int e = L.d.z + k * L.d.y + lane, f = P.face[back][e];
                 if (f < 0) break;
-                const double xk = await(hand, P.pos[back][e], want);
+                const double xk = awaitValue<double>(hand, P.pos[back][e], want);
                 if (Factor)
                     v -= upper[f] * lower[f] / xk;
                 else
                     v -= rd * (back ? upper[f] : lower[f]) * xk;
             }
-            put(hand, own, want, v);
+            Hand<double>::put(hand, own, want, v);
             if (Factor)
                 out[L.c] = 1.0 / v;
             else if (back)
@@ -586,9 +525,9 @@ __global__ __launch_bounds__(64) void flowGsK(int nSteps, const int4* __restrict
                                               const int* __restrict__ self, const int* __restrict__ face,
                                               const int* __restrict__ pos, const double* __restrict__ diag,
                                               const double* __restrict__ upper, const double* __restrict__ b,
-                                              double* psi, double* bPrime, unsigned long long* hand, unsigned* state)
+                                              double* psi, double* bPrime, Word* hand, unsigned* state)
 {
-    const unsigned tag = __hip_atomic_load(state + kTag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    const unsigned tag = launchTag(state);
     const int lane = threadIdx.x;
     for (int t = takeChunk(state); t < nSteps; t = takeChunk(state))
     {
@@ -617,7 +556,7 @@ __global__ __launch_bounds__(64) void flowGsK(int nSteps, const int4* __restrict
                 for (int k = L.d.w - 1; k >= W; --k)
                 {
                     const int e = L.d.z + k * L.d.y + lane, f = face[e];
-                    if (f >= 0) v -= upper[f] * await(hand, pos[e], tag);
+                    if (f >= 0) v -= upper[f] * awaitValue<double>(hand, pos[e], tag);
                 }
 #pragma unroll
                 for (int k = W - 1; k >= 0; --k)
@@ -637,13 +576,13 @@ __global__ __launch_bounds__(64) void flowGsK(int nSteps, const int4* __restrict
                 {
                     const int e = L.d.z + k * L.d.y + lane, f = face[e];
                     if (f < 0) break;
-                    v -= upper[f] * (k < nl ? await(hand, pos[e], tag) : psi[pos[e]]);
+                    v -= upper[f] * (k < nl ? awaitValue<double>(hand, pos[e], tag) : psi[pos[e]]);
                     if (bPrime && k + 1 == nl) bPrime[L.c] = v;
                 }
             }
             v /= dg;
             psi[L.c] = v;
-            put(hand, own, tag, v);
+            Hand<double>::put(hand, own, tag, v);
         }
     }
     leave(state, tag, 1);
@@ -803,7 +742,7 @@ bool planBuild(Ctx& c, Mesh& m, SweepPlan* p)
         p->dFwd.resize(n);
         return true;
     }
-    p->hand.upload(std::vector<unsigned long long>(2 * (size_t)n, 0ull), c.stream);
+    p->hand.upload(std::vector<Word>(2 * (size_t)n, 0ull), c.stream);
     p->state.upload(std::vector<unsigned>{0u, 0u, 1u}, c.stream);
     return true;
 }
@@ -915,8 +854,8 @@ template <int W, bool Factor>
 void substFlow(Ctx& c, SweepPlan& p, const double* diag, const double* upper, const double* lower, const double* rD,
                const double* r, double* out, const int* stop)
 {
-    const int chunks = p.fwd.nSteps + (Factor ? 0 : p.bwd.nSteps);
-    flowSubstK<W, Factor><<<std::min(chunks, kFlowWaves), 64, 0, c.stream>>>(flowView(p), diag, upper, lower, rD, r, out,
+    const int steps = p.fwd.nSteps + (Factor ? 0 : p.bwd.nSteps);
+    flowSubstK<W, Factor><<<std::min(steps, kFlowWaves), 64, 0, c.stream>>>(flowView(p), diag, upper, lower, rD, r, out,
                                                                            p.hand.p, p.state.p, stop);
 }
 

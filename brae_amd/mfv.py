@@ -520,7 +520,7 @@ class Amg:
 
     def coarse_mode(self, mode=-1):
         """sets how the coarsest grids run (0 per-grid kernels, 1 one workgroup, 2 one workgroup with the
-        coarsest grids staged in LDS; -1 leaves it) and returns (the tail's first grid, the first grid
+        coarsest grids staged in LDS; -1 leaves it; until a mode is set, one launch of many workgroups) and returns (the tail's first grid, the first grid
         staged, the LDS bytes the staged grids take)"""
         t, g, b = ctypes.c_int(), ctypes.c_int(), ctypes.c_int()
         self.ctx._check(lib().mfv_amg_coarse_mode(self.h, mode, ctypes.byref(t), ctypes.byref(g), ctypes.byref(b)),

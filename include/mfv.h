@@ -342,11 +342,13 @@ int mfv_amg_grid_size(mfv_amg amg, int grid, int* nCells, int* nFaces);
  * offsets. 0 offsets: the fine matrix is read as sliced rows. */
 int mfv_amg_fine_stencil(mfv_amg amg, int* nOffsets, int* hOffsets);
 /* How the coarsest grids' cycle runs, no counterpart in the reference (its small levels run one kernel
- * per step). Below 4096 cells the grids from the first such one down run in one workgroup (the tail):
- * mode 2 (default) stages the tail's coarsest grids -- as many as fit the device's LDS per workgroup --
- * in that workgroup's LDS and reads the others where they are; mode 1 reads them all where they are;
- * mode 0 runs every grid with its own kernels. All modes give the same bits (the scaled correction
- * keeps mode 1's kernel). mode -1 only queries. *tailStart: the tail's first grid (0: no tail);
+ * per step). Until a mode is set, the grids from the first one of at most 8192 cells down run in one
+ * launch of many workgroups that hand the steps' values on to each other. The modes below 4096 cells
+ * run the grids from the first such one down in one workgroup (the tail): mode 2 stages the tail's
+ * coarsest grids -- as many as fit the device's LDS per workgroup -- in that workgroup's LDS and reads
+ * the others where they are; mode 1 reads them all where they are; mode 0 runs every grid with its own
+ * kernels. All give the same bits, except that the scaled correction keeps mode 1's kernel in mode 2
+ * and takes its sums in another order until a mode is set. mode -1 only queries. *tailStart: the tail's first grid (0: no tail);
  * *ldsGrid: the first grid staged (0: none); *ldsBytes: the LDS the staged grids take, in the precision
  * of the last mfv_amg_galerkin; any of the three may be NULL. */
 int mfv_amg_coarse_mode(mfv_amg amg, int mode, int* tailStart, int* ldsGrid, int* ldsBytes);
