@@ -752,6 +752,9 @@ __global__ __launch_bounds__(kTpb) void zeroK(int n, double* __restrict__ x)
 // bc value; zeroGradient: the cell value), over V. Each face's weight, area vector and neighbour index are
 // loaded once for all NC components. Writes each component's gradient xyz per cell (g3) and, when g9 is
 // given, the packed tensor g9[(i*3 + k)*n + c] = d(psi_k)/dx_i.
+// Bound by the face data's HBM reads, once a cell's loads are in flight together (the first kBatch faces of each run,
+// as in matrixH3K); face after face it was the chain of their latencies: 41 -> 28 us at 640 k cells, 358 -> 259 at
+// 5.3 M (3.8 TB/s), one component.
 struct Grad3Args
 {
     const double* psi[3];
@@ -783,33 +786,63 @@ __global__ __launch_bounds__(kTpb) void gradGauss3K(int n, SlabPart part, int nF
         gy[j] = 0.0;
         gz[j] = 0.0;
     }
-    for (int k = losortStart[c]; k < losortStart[c + 1]; ++k)
-    {
-        const int f = losort[k], o = losortOwner[k];
-        const double wf = w[f], sx = Sf[3 * (size_t)f], sy = Sf[3 * (size_t)f + 1], sz = Sf[3 * (size_t)f + 2];
+    const int l0 = losortStart[c], l1 = losortStart[c + 1];
+    const int f0 = ownerStart[c], f1 = ownerStart[c + 1];
+    auto add = [&](bool owned, double wf, double sx, double sy, double sz, const double (&po)[NC]) {
 #pragma unroll
         for (int j = 0; j < NC; ++j)
         {
-            const double pf = wf * (a.psi[j][o] - pc[j]) + pc[j];
-            gx[j] = gx[j] - sx * pf;
-            gy[j] = gy[j] - sy * pf;
-            gz[j] = gz[j] - sz * pf;
+            const double pf = owned ? wf * (pc[j] - po[j]) + po[j] : wf * (po[j] - pc[j]) + pc[j];
+            gx[j] = owned ? gx[j] + sx * pf : gx[j] - sx * pf;
+            gy[j] = owned ? gy[j] + sy * pf : gy[j] - sy * pf;
+            gz[j] = owned ? gz[j] + sz * pf : gz[j] - sz * pf;
         }
-    }
-    for (int f = ownerStart[c]; f < ownerStart[c + 1]; ++f)
+    };
+    double wl[kBatch] = {}, sl[kBatch][3] = {}, pl[kBatch][NC] = {};
+    double wo[kBatch] = {}, so[kBatch][3] = {}, po[kBatch][NC] = {};
+    if (nF > 0)   // uniform
     {
-        const int nb = neighbour[f];
-        const double wf = w[f], sx = Sf[3 * (size_t)f], sy = Sf[3 * (size_t)f + 1], sz = Sf[3 * (size_t)f + 2];
+        const int last = nF - 1;
+        int lf[kBatch], lo[kBatch], nb[kBatch];
 #pragma unroll
-        for (int j = 0; j < NC; ++j)
+        for (int u = 0; u < kBatch; ++u)
         {
-            const double pn = a.psi[j][nb];
-            const double pf = wf * (pc[j] - pn) + pn;
-            gx[j] = gx[j] + sx * pf;
-            gy[j] = gy[j] + sy * pf;
-            gz[j] = gz[j] + sz * pf;
+            const int j = min(l0 + u, last), f = min(f0 + u, last);
+            lf[u] = losort[j];
+            lo[u] = losortOwner[j];
+            nb[u] = neighbour[f];
+            wo[u] = w[f];
+#pragma unroll
+            for (int i = 0; i < 3; ++i) so[u][i] = Sf[3 * (size_t)f + i];
+        }
+#pragma unroll
+        for (int u = 0; u < kBatch; ++u)
+        {
+            wl[u] = w[lf[u]];
+#pragma unroll
+            for (int i = 0; i < 3; ++i) sl[u][i] = Sf[3 * (size_t)lf[u] + i];
+#pragma unroll
+            for (int j = 0; j < NC; ++j)
+            {
+                pl[u][j] = a.psi[j][lo[u]];
+                po[u][j] = a.psi[j][nb[u]];
+            }
         }
     }
+#pragma unroll
+    for (int u = 0; u < kBatch; ++u)
+        if (l0 + u < l1) add(false, wl[u], sl[u][0], sl[u][1], sl[u][2], pl[u]);
+    auto one = [&](bool owned, int f, int other) {
+        double p[NC];
+#pragma unroll
+        for (int j = 0; j < NC; ++j) p[j] = a.psi[j][other];
+        add(owned, w[f], Sf[3 * (size_t)f], Sf[3 * (size_t)f + 1], Sf[3 * (size_t)f + 2], p);
+    };
+    for (int k = l0 + kBatch; k < l1; ++k) one(false, losort[k], losortOwner[k]);
+#pragma unroll
+    for (int u = 0; u < kBatch; ++u)
+        if (f0 + u < f1) add(true, wo[u], so[u][0], so[u][1], so[u][2], po[u]);
+    for (int f = f0 + kBatch; f < f1; ++f) one(true, f, neighbour[f]);
     for (int k = bndStart[c]; k < bndStart[c + 1]; ++k)
     {
         const int i = bndFaces[k];
