@@ -442,7 +442,10 @@ __global__ __launch_bounds__(kTpb) void dev2tK(int n, const double* __restrict__
 // tensorDivKernel): per cell, its internal faces in face order -- the losort run subtracted, the owned
 // run added -- with T_f = w*T_own + (1-w)*T_nei and (Sf & T_f)_j = Sx*T_xj + Sy*T_yj + Sz*T_zj, then its
 // boundary faces not marked empty, Sf_b & T_b added. The cell's own tensor stays in registers; the
-// other cell's tensor, w and Sf of up to kBatch faces are loaded together (clamped indices).
+// other cell's tensor, w and Sf of up to kBatch faces are loaded together (clamped indices). Bound by the latency
+// of those loads: three waves per SIMD with the registers to keep a batch in flight take 178 us at 2 M cells and 57
+// at 640 k, where the compiler's own choice of four split the batches (218 and 69); two waves 191; two lanes a
+// cell, a run each, 88 at 640 k.
 __device__ __forceinline__ void tensorFaceFlux(double wf, bool selfOwns, const double (&ts)[9],
                                                const double (&to)[9], double sx, double sy, double sz,
                                                double (&r)[3])
@@ -479,19 +482,13 @@ __device__ __forceinline__ void loadTensor(int n, int cell, const double* __rest
 }
 
 template <bool Slab, bool FromGrad>
-__global__ __launch_bounds__(kTpb) void tensorDivK(int n, SlabPart part, int nF, int nB,
-                                                   const label* __restrict__ ownerStart,
-                                                   const label* __restrict__ losortStart,
-                                                   const label* __restrict__ losort,
-                                                   const label* __restrict__ losortOwner,
-                                                   const label* __restrict__ neighbour,
-                                                   const label* __restrict__ bndStart,
-                                                   const label* __restrict__ bndFaces,
-                                                   const int* __restrict__ isEmpty, const double* __restrict__ w,
-                                                   const double* __restrict__ Sf, const double* __restrict__ Tc,
-                                                   const double* __restrict__ nu, const double* __restrict__ Tb,
-                                                   double* __restrict__ dX,
-                                                   double* __restrict__ dY, double* __restrict__ dZ)
+__global__ __launch_bounds__(kTpb) __attribute__((amdgpu_waves_per_eu(2, 3))) void tensorDivK(
+    int n, SlabPart part, int nF, int nB, const label* __restrict__ ownerStart, const label* __restrict__ losortStart,
+    const label* __restrict__ losort, const label* __restrict__ losortOwner, const label* __restrict__ neighbour,
+    const label* __restrict__ bndStart, const label* __restrict__ bndFaces, const int* __restrict__ isEmpty,
+    const double* __restrict__ w, const double* __restrict__ Sf, const double* __restrict__ Tc,
+    const double* __restrict__ nu, const double* __restrict__ Tb, double* __restrict__ dX, double* __restrict__ dY,
+    double* __restrict__ dZ)
 {
     const int c = gatherCell<Slab>(n, part);
     if (c < 0) return;
