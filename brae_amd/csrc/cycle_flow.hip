@@ -358,20 +358,11 @@ __global__ __launch_bounds__(kThreads) void flowCycleK(const FlowGrid* __restric
         const bool lead = lane % kLanes == 0;   // the lane that writes its row's value
         const FlowGrid& G = grids[g];
         const Tv m = G.xm ? (Tv)*G.xm : Tv(1), im = G.xm ? (Tv)(1.0f / *G.xm) : Tv(1);
-        // a finished value: to the finer grid of this launch, or out of it
+        Tv done = Tv(0);         // a finished value, handed on below
+        bool finished = false;
         auto finish = [&](Tv v) {
-            if (!lead) return;
-            if (g > 0)
-            {
-                Hand<Tv>::put(G.f, c, tag, v);
-                return;
-            }
-            if (out)
-            {
-                const CycVec<Tv, Ts> XO(out, G.xm);
-                XO.set(c, v);
-            }
-            up(c, v);
+            done = v;
+            finished = true;
         };
         // before a step on the way up: what the next grid's last step waited for
         auto gateUp = [&](int mc) {
@@ -588,6 +579,21 @@ __global__ __launch_bounds__(kThreads) void flowCycleK(const FlowGrid* __restric
                     Hand<Tv>::put(G.y[0], c, tag, stored<Tv, Ts>(xo, m, im));
                 else if (!st.nExtra)
                     finish(xo);
+            }
+        }
+        // to the finer grid of this launch, or out of it (once for every kind of step: the kernel's size costs it)
+        if (finished && lead)
+        {
+            if (g > 0)
+                Hand<Tv>::put(G.f, c, tag, done);
+            else
+            {
+                if (out)
+                {
+                    const CycVec<Tv, Ts> XO(out, G.xm);
+                    XO.set(c, done);
+                }
+                up(c, done);
             }
         }
     }

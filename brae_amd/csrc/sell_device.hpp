@@ -221,7 +221,9 @@ struct CycVec<float, __half>
 
 // The coarse-to-fine injection, fused into whichever kernel finishes a coarse grid's cycle: coarse cell
 // C's final value goes to every fine cell of its agglomerate (the fine grid's cellStart/cellList), so
-// the fine grid reads its correction e = xc[map] as a plain vector (prolongT's values, written once).
+// the fine grid reads its correction e = xc[map] as a plain vector (prolongT's values, written once). The cells go
+// by records of four (see restrictK), the first one asked for ahead: prolongSmoothK on 522 k, 129 k and 32 k rows
+// 21.1, 10.5 and 8.6 us through the lists, 18.8, 9.2 and 7.3.
 template <typename Tv, typename Ts>
 struct Scatter
 {
@@ -229,21 +231,23 @@ struct Scatter
     const int* __restrict__ list;
     Ts* __restrict__ e;        // null: no fine grid waits for this one (grid 0)
     const float* xm;           // the fine grid's multiplier
-    const int4* quads;         // the fine grid's agglomerates of up to four (may be null: the lists alone)
-    __device__ void operator()(int C, Tv v) const
+    const int4* quads;         // the fine grid's agglomerates as records (may be null: the lists)
+    // cell C's first record, for a caller that asks for it before its value is there
+    __device__ int4 first(int C) const { return e && quads ? quads[C] : int4{-1, -1, -1, -1}; }
+    __device__ void operator()(int C, Tv v) const { (*this)(C, v, first(C)); }
+    __device__ void operator()(int C, Tv v, int4 q) const
     {
         if (!e) return;
         const CycVec<Tv, Ts> E(e, xm);
         if (quads)
         {
-            const int4 q = quads[C];
-            if (q.x >= 0)
+            for (;; q = quads[-2 - q.w])
             {
-                E.set(q.x, v);
+                if (q.x >= 0) E.set(q.x, v);
                 if (q.y >= 0) E.set(q.y, v);
                 if (q.z >= 0) E.set(q.z, v);
                 if (q.w >= 0) E.set(q.w, v);
-                return;
+                if (q.w >= -1) return;
             }
         }
         for (int k = start[C]; k < start[C + 1]; ++k) E.set(list[k], v);
