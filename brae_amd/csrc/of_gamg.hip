@@ -16,6 +16,7 @@
 // the host instead; here nothing leaves the device. A coarsest level too big for LDS runs the
 // multi-launch guarded PCG-DIC.
 #include "amg.hpp"
+#include "reduce.hpp"
 
 #include <algorithm>
 #include <cmath>
@@ -33,6 +34,7 @@ constexpr double kGreat = 1e20;      // GREAT
 constexpr int kCoarsestMaxIter = 1000;
 constexpr int kCoarsestLanes = 64;
 constexpr size_t kCoarsestLds = 60 * 1024;
+constexpr int kScaleParts = 256;     // partials that the scaling's update finishes itself (see Cycle::scale)
 
 // device scalars of a solve
 enum : int { S_NF = 0, S_SUMMAG, S_RHO, S_RHOOLD, S_PQ, S_NUM, S_DEN, S_CINIT, S_CFINAL, S_CITER, S_COUNT = 16 };
@@ -58,16 +60,63 @@ __global__ __launch_bounds__(kTpb) void prolongK(int nf, const int* __restrict__
 }
 
 // GAMGSolver::scale's update (gamg_solver_cpp.cu:386-407): sf = (x.b)/(x.Ax +- VSMALL),
-// x = sf*x + (b - sf*Ax)/D
+// x = sf*x + (b - sf*Ax)/D; with nParts > 0 every workgroup finishes the two sums from their partials, else st has them
 __global__ __launch_bounds__(kTpb) void scaleApplyK(int n, double* __restrict__ field, const double* __restrict__ Acf,
                                                     const double* __restrict__ source,
-                                                    const double* __restrict__ diag, const double* __restrict__ st)
+                                                    const double* __restrict__ diag, const double* __restrict__ st,
+                                                    int nParts, const double* __restrict__ pn,
+                                                    const double* __restrict__ pd)
 {
+    static_assert(kTpb == kReduceBlock, "the sums are finished by kReduceBlock-thread workgroups");
+    __shared__ double lds[2 * (kFinishBlock / 64)];
+    __shared__ double shNum, shDen;
+    if (nParts > 0)
+    {
+        double num, den;
+        finish2InBlock(nParts, pn, pd, lds, num, den);
+        if (threadIdx.x == 0)
+        {
+            shNum = num;
+            shDen = den;
+        }
+        __syncthreads();
+    }
     const int i = blockIdx.x * kTpb + threadIdx.x;
     if (i >= n) return;
-    const double num = st[S_NUM], den = st[S_DEN];
+    const double num = nParts > 0 ? shNum : st[S_NUM], den = nParts > 0 ? shDen : st[S_DEN];
     const double sf = num / (den >= 0 ? den + kVSmall : den - kVSmall);
     field[i] = sf * field[i] + (source[i] - sf * Acf[i]) / diag[i];
+}
+
+// A field on a level with the two sums of its scaling, field.source and field.(A field), a partial of each per
+// workgroup, in amulK's and dotK's arithmetic
+__global__ __launch_bounds__(kReduceBlock) void amulDotsK(int n, const label* __restrict__ ownerStart,
+                                                          const label* __restrict__ losortStart,
+                                                          const label* __restrict__ losort,
+                                                          const label* __restrict__ losortOwner,
+                                                          const label* __restrict__ neighbour, LduView A,
+                                                          const double* __restrict__ x,
+                                                          const double* __restrict__ source, double* __restrict__ Ax,
+                                                          double* __restrict__ pn, double* __restrict__ pd)
+{
+    __shared__ double lds[kReduceBlock / 64];
+    double num = 0.0, den = 0.0;
+    MFV_ROWS(n, c)
+    {
+        const double xc = x[c];
+        double s = A.diag[c] * xc;
+        for (int k = losortStart[c]; k < losortStart[c + 1]; ++k) s += A.lower[losort[k]] * x[losortOwner[k]];
+        for (int f = ownerStart[c]; f < ownerStart[c + 1]; ++f) s += A.upper[f] * x[neighbour[f]];
+        Ax[c] = s;
+        num += xc * source[c];
+        den += xc * s;
+    }
+    const double sn = blockSum(num, lds), sd = blockSum(den, lds);
+    if (threadIdx.x == 0)
+    {
+        pn[blockIdx.x] = sn;
+        pd[blockIdx.x] = sd;
+    }
 }
 
 __global__ __launch_bounds__(kTpb) void fillK(int n, double v, double* __restrict__ x)
@@ -509,13 +558,33 @@ private:
         scaleRefApplyK<<<blocks(n), kTpb, 0, c_.stream>>>(n, field, Acf, source, L.A.diag, w_.st.p);
     }
 
+    // On levels of a few hundred to a few thousand cells launches are the cost: the product and its two sums in one,
+    // the sums finished by the update's workgroups, so two launches where six were: a solve over 13,861 cells 42.5
+    // -> 40.8 ms (41.5 with the finishing launches kept). Above kScaleParts partials, which every workgroup would
+    // read, two finishing launches come in between; at 65 k to 590 k cells neither way is the faster.
     void scale(Level& L, double* field, double* Acf, const double* source)
     {
-        const int n = L.A.nCells;
-        launchAmul(c_, *L.m, L.A, field, Acf);
-        launchDot(c_, n, field, source, w_.st.p + S_NUM, 0);
-        launchDot(c_, n, field, Acf, w_.st.p + S_DEN, 1);
-        scaleApplyK<<<blocks(n), kTpb, 0, c_.stream>>>(n, field, Acf, source, L.A.diag, w_.st.p);
+        const Mesh& m = *L.m;
+        const int n = L.A.nCells, g = reduceGrid(n);
+        double *pn = c_.partials.p, *pd = c_.partials.p + (size_t)kMaxReduceBlocks;
+        if (c_.sequentialReduce)
+        {
+            launchAmul(c_, m, L.A, field, Acf);
+            launchDot(c_, n, field, source, w_.st.p + S_NUM, 0);
+            launchDot(c_, n, field, Acf, w_.st.p + S_DEN, 1);
+        }
+        else
+        {
+            amulDotsK<<<g, kReduceBlock, 0, c_.stream>>>(n, m.ownerStart.p, m.losortStart.p, m.losort.p, m.losortOwner.p,
+                                                         m.neighbour.p, L.A, field, source, Acf, pn, pd);
+            if (g > kScaleParts)
+            {
+                finishK<<<1, kFinishBlock, 0, c_.stream>>>(g, pn, StoreTo{w_.st.p + S_NUM}, nullptr);
+                finishK<<<1, kFinishBlock, 0, c_.stream>>>(g, pd, StoreTo{w_.st.p + S_DEN}, nullptr);
+            }
+        }
+        const bool inBlock = !c_.sequentialReduce && g <= kScaleParts;
+        scaleApplyK<<<blocks(n), kTpb, 0, c_.stream>>>(n, field, Acf, source, L.A.diag, w_.st.p, inBlock ? g : 0, pn, pd);
     }
 
     void coarsestSolve()
