@@ -17,8 +17,84 @@ constexpr int kTpb = 256;
 
 inline int blocks(int n) { return (n + kTpb - 1) / kTpb; }
 
+// A cell's faces, first the ones it is the neighbour of, then its own, both ascending: fn(value, owned) per face in
+// that order, its value from aNei or aOwn. The first kBatch of each run are loaded together, with clamped indices,
+// and dropped past the run's end; the rest follow one by one. Face after face the loads' latencies added up
+// (what remains is HBM time: the sums of a face field at 2 M cells 37, 32 and 30 us -> 30, 28 and 26, at 5.3 M 82 ->
+// 68; the rows at 640 k cells 18.2 -> 15.2, at 4,096 5.9, 3.6 and 3.3 -> 4.9, 3.1 and 2.9).
+constexpr int kBatch = 3;
+
+template <typename Fn>
+__device__ __forceinline__ void cellFaces(int c, int nF, const label* __restrict__ ownerStart,
+                                          const label* __restrict__ losortStart, const label* __restrict__ losort,
+                                          const double* __restrict__ aNei, const double* __restrict__ aOwn, Fn fn)
+{
+    const int l0 = losortStart[c], l1 = losortStart[c + 1], o0 = ownerStart[c], o1 = ownerStart[c + 1];
+    double vl[kBatch] = {}, vo[kBatch] = {};
+    if (nF > 0)   // uniform
+    {
+        int lf[kBatch];
+#pragma unroll
+        for (int u = 0; u < kBatch; ++u)
+        {
+            lf[u] = losort[min(l0 + u, nF - 1)];
+            vo[u] = aOwn[min(o0 + u, nF - 1)];
+        }
+#pragma unroll
+        for (int u = 0; u < kBatch; ++u) vl[u] = aNei[lf[u]];
+    }
+#pragma unroll
+    for (int u = 0; u < kBatch; ++u)
+        if (l0 + u < l1) fn(vl[u], false);
+    for (int k = l0 + kBatch; k < l1; ++k) fn(aNei[losort[k]], false);
+#pragma unroll
+    for (int u = 0; u < kBatch; ++u)
+        if (o0 + u < o1) fn(vo[u], true);
+    for (int f = o0 + kBatch; f < o1; ++f) fn(aOwn[f], true);
+}
+
+// The same with a matrix row's operands: fn(coefficient, x at the face's other cell)
+template <typename Fn>
+__device__ __forceinline__ void rowFaces(int c, int nF, const label* __restrict__ ownerStart,
+                                         const label* __restrict__ losortStart, const label* __restrict__ losort,
+                                         const label* __restrict__ losortOwner, const label* __restrict__ neighbour,
+                                         const double* __restrict__ upper, const double* __restrict__ lower,
+                                         const double* __restrict__ x, Fn fn)
+{
+    const int l0 = losortStart[c], l1 = losortStart[c + 1], o0 = ownerStart[c], o1 = ownerStart[c + 1];
+    double al[kBatch] = {}, au[kBatch] = {}, xl[kBatch] = {}, xu[kBatch] = {};
+    if (nF > 0)   // uniform
+    {
+        int lf[kBatch], lc[kBatch], uc[kBatch];
+#pragma unroll
+        for (int u = 0; u < kBatch; ++u)
+        {
+            const int k = min(l0 + u, nF - 1), f = min(o0 + u, nF - 1);
+            lf[u] = losort[k];
+            lc[u] = losortOwner[k];
+            uc[u] = neighbour[f];
+            au[u] = upper[f];
+        }
+#pragma unroll
+        for (int u = 0; u < kBatch; ++u)
+        {
+            al[u] = lower[lf[u]];
+            xl[u] = x[lc[u]];
+            xu[u] = x[uc[u]];
+        }
+    }
+#pragma unroll
+    for (int u = 0; u < kBatch; ++u)
+        if (l0 + u < l1) fn(al[u], xl[u]);
+    for (int k = l0 + kBatch; k < l1; ++k) fn(lower[losort[k]], x[losortOwner[k]]);
+#pragma unroll
+    for (int u = 0; u < kBatch; ++u)
+        if (o0 + u < o1) fn(au[u], xu[u]);
+    for (int f = o0 + kBatch; f < o1; ++f) fn(upper[f], x[neighbour[f]]);
+}
+
 // y = A x (ldu_spmv.cu:5-24, device_spmv.cu:16-58)
-__global__ __launch_bounds__(kTpb) void amulK(int n, const label* __restrict__ ownerStart,
+__global__ __launch_bounds__(kTpb) void amulK(int n, int nF, const label* __restrict__ ownerStart,
                                               const label* __restrict__ losortStart,
                                               const label* __restrict__ losort,
                                               const label* __restrict__ losortOwner,
@@ -29,15 +105,13 @@ __global__ __launch_bounds__(kTpb) void amulK(int n, const label* __restrict__ o
     const int c = xcdBlock() * kTpb + threadIdx.x;
     if (c >= n) return;
     double s = diag[c] * x[c];
-    const int l0 = losortStart[c], l1 = losortStart[c + 1];
-    for (int k = l0; k < l1; ++k) s += lower[losort[k]] * x[losortOwner[k]];
-    const int o0 = ownerStart[c], o1 = ownerStart[c + 1];
-    for (int f = o0; f < o1; ++f) s += upper[f] * x[neighbour[f]];
+    rowFaces(c, nF, ownerStart, losortStart, losort, losortOwner, neighbour, upper, lower, x,
+             [&](double a, double v) { s += a * v; });
     y[c] = s;
 }
 
 // r = b - A x, term by term (gamg_solver_cpp.cu:88-112)
-__global__ __launch_bounds__(kTpb) void residualK(int n, const label* __restrict__ ownerStart,
+__global__ __launch_bounds__(kTpb) void residualK(int n, int nF, const label* __restrict__ ownerStart,
                                                   const label* __restrict__ losortStart,
                                                   const label* __restrict__ losort,
                                                   const label* __restrict__ losortOwner,
@@ -49,10 +123,8 @@ __global__ __launch_bounds__(kTpb) void residualK(int n, const label* __restrict
     const int c = xcdBlock() * kTpb + threadIdx.x;
     if (c >= n) return;
     double s = b[c] - diag[c] * x[c];
-    const int l0 = losortStart[c], l1 = losortStart[c + 1];
-    for (int k = l0; k < l1; ++k) s -= lower[losort[k]] * x[losortOwner[k]];
-    const int o0 = ownerStart[c], o1 = ownerStart[c + 1];
-    for (int f = o0; f < o1; ++f) s -= upper[f] * x[neighbour[f]];
+    rowFaces(c, nF, ownerStart, losortStart, losort, losortOwner, neighbour, upper, lower, x,
+             [&](double a, double v) { s -= a * v; });
     r[c] = s;
 }
 
@@ -81,7 +153,7 @@ struct NormPost
     __device__ void operator()(double s) const { *out = s + 1e-20; }
 };
 
-__device__ __forceinline__ double normSummand(int c, const label* __restrict__ ownerStart,
+__device__ __forceinline__ double normSummand(int c, int nF, const label* __restrict__ ownerStart,
                                               const label* __restrict__ losortStart, const label* __restrict__ losort,
                                               const label* __restrict__ losortOwner,
                                               const label* __restrict__ neighbour, const double* __restrict__ diag,
@@ -91,25 +163,16 @@ __device__ __forceinline__ double normSummand(int c, const label* __restrict__ o
 {
     double ax = diag[c] * psi[c];
     double sa = diag[c];
-    const int l0 = losortStart[c], l1 = losortStart[c + 1];
-    for (int k = l0; k < l1; ++k)
-    {
-        const double lo = lower[losort[k]];
-        ax += lo * psi[losortOwner[k]];
-        sa += lo;
-    }
-    const int o0 = ownerStart[c], o1 = ownerStart[c + 1];
-    for (int f = o0; f < o1; ++f)
-    {
-        ax += upper[f] * psi[neighbour[f]];
-        sa += upper[f];
-    }
+    rowFaces(c, nF, ownerStart, losortStart, losort, losortOwner, neighbour, upper, lower, psi, [&](double a, double v) {
+        ax += a * v;
+        sa += a;
+    });
     const double t = sa * xRef;
     return fabs(ax - t) + fabs(b[c] - t);
 }
 
 __global__ __launch_bounds__(kReduceBlock) void normFactorK(
-    int n, const label* __restrict__ ownerStart, const label* __restrict__ losortStart,
+    int n, int nF, const label* __restrict__ ownerStart, const label* __restrict__ losortStart,
     const label* __restrict__ losort, const label* __restrict__ losortOwner, const label* __restrict__ neighbour,
     const double* __restrict__ diag, const double* __restrict__ upper, const double* __restrict__ lower,
     const double* __restrict__ psi, const double* __restrict__ b, const double* __restrict__ sumPsi,
@@ -119,11 +182,11 @@ __global__ __launch_bounds__(kReduceBlock) void normFactorK(
     const double xRef = *sumPsi / (double)n;
     double v = 0.0;
     MFV_ROWS(n, c)
-    v += normSummand(c, ownerStart, losortStart, losort, losortOwner, neighbour, diag, upper, lower, psi, b, xRef);
+    v += normSummand(c, nF, ownerStart, losortStart, losort, losortOwner, neighbour, diag, upper, lower, psi, b, xRef);
     storePartial(blockSum(v, lds), partials);
 }
 
-__global__ void normFactorSeqK(int n, const label* __restrict__ ownerStart, const label* __restrict__ losortStart,
+__global__ void normFactorSeqK(int n, int nF, const label* __restrict__ ownerStart, const label* __restrict__ losortStart,
                                const label* __restrict__ losort, const label* __restrict__ losortOwner,
                                const label* __restrict__ neighbour, const double* __restrict__ diag,
                                const double* __restrict__ upper, const double* __restrict__ lower,
@@ -134,7 +197,7 @@ __global__ void normFactorSeqK(int n, const label* __restrict__ ownerStart, cons
     const double xRef = *sumPsi / (double)n;
     double s = 0.0;
     for (int c = 0; c < n; ++c)
-        s += normSummand(c, ownerStart, losortStart, losort, losortOwner, neighbour, diag, upper, lower, psi, b, xRef);
+        s += normSummand(c, nF, ownerStart, losortStart, losort, losortOwner, neighbour, diag, upper, lower, psi, b, xRef);
     *out = s + 1e-20;
 }
 
@@ -151,7 +214,7 @@ __global__ __launch_bounds__(kTpb) void lapFaceK(int nF, const double* __restric
 }
 
 // diag = -(sum of coefficients) in face order (fvm.cuh:148-149, device_fvm.cu:235-273)
-__global__ __launch_bounds__(kTpb) void lapDiagK(int n, const label* __restrict__ ownerStart,
+__global__ __launch_bounds__(kTpb) void lapDiagK(int n, int nF, const label* __restrict__ ownerStart,
                                                  const label* __restrict__ losortStart,
                                                  const label* __restrict__ losort, const double* __restrict__ upper,
                                                  double* __restrict__ diag)
@@ -159,10 +222,7 @@ __global__ __launch_bounds__(kTpb) void lapDiagK(int n, const label* __restrict_
     const int c = xcdBlock() * kTpb + threadIdx.x;
     if (c >= n) return;
     double d = 0.0;
-    const int l0 = losortStart[c], l1 = losortStart[c + 1];
-    for (int k = l0; k < l1; ++k) d -= upper[losort[k]];
-    const int o0 = ownerStart[c], o1 = ownerStart[c + 1];
-    for (int f = o0; f < o1; ++f) d -= upper[f];
+    cellFaces(c, nF, ownerStart, losortStart, losort, upper, upper, [&](double u, bool) { d -= u; });
     diag[c] = d;
 }
 
@@ -218,7 +278,7 @@ __global__ __launch_bounds__(kTpb) void divFaceLinearK(int nF, const double* __r
 }
 
 // diag -= lower (owned faces), -= upper (neighbour faces), in face order
-__global__ __launch_bounds__(kTpb) void divDiagK(int n, const label* __restrict__ ownerStart,
+__global__ __launch_bounds__(kTpb) void divDiagK(int n, int nF, const label* __restrict__ ownerStart,
                                                  const label* __restrict__ losortStart,
                                                  const label* __restrict__ losort, const double* __restrict__ upper,
                                                  const double* __restrict__ lower, double* __restrict__ diag)
@@ -226,10 +286,7 @@ __global__ __launch_bounds__(kTpb) void divDiagK(int n, const label* __restrict_
     const int c = xcdBlock() * kTpb + threadIdx.x;
     if (c >= n) return;
     double d = 0.0;
-    const int l0 = losortStart[c], l1 = losortStart[c + 1];
-    for (int k = l0; k < l1; ++k) d -= upper[losort[k]];
-    const int o0 = ownerStart[c], o1 = ownerStart[c + 1];
-    for (int f = o0; f < o1; ++f) d -= lower[f];
+    cellFaces(c, nF, ownerStart, losortStart, losort, upper, lower, [&](double u, bool) { d -= u; });
     diag[c] = d;
 }
 
@@ -310,7 +367,7 @@ __global__ __launch_bounds__(kTpb) void interpK(int nF, int nB, const label* __r
 
 // source += sign * (div(phi) * V) with div = (sum_own phi - sum_nei phi + sum_boundary phi_b)/V in face
 // order (fvc.cu:706-730; pEqn_cpp.cu:238-242)
-__global__ __launch_bounds__(kTpb) void divSourceK(int n, const label* __restrict__ ownerStart,
+__global__ __launch_bounds__(kTpb) void divSourceK(int n, int nF, const label* __restrict__ ownerStart,
                                                    const label* __restrict__ losortStart,
                                                    const label* __restrict__ losort,
                                                    const label* __restrict__ bndStart,
@@ -321,10 +378,7 @@ __global__ __launch_bounds__(kTpb) void divSourceK(int n, const label* __restric
     const int c = xcdBlock() * kTpb + threadIdx.x;
     if (c >= n) return;
     double d = 0.0;
-    const int l0 = losortStart[c], l1 = losortStart[c + 1];
-    for (int k = l0; k < l1; ++k) d -= phi[losort[k]];
-    const int o0 = ownerStart[c], o1 = ownerStart[c + 1];
-    for (int f = o0; f < o1; ++f) d += phi[f];
+    cellFaces(c, nF, ownerStart, losortStart, losort, phi, phi, [&](double p, bool owned) { d = owned ? d + p : d - p; });
     if (phib)
         for (int k = bndStart[c]; k < bndStart[c + 1]; ++k) d += phib[bndFaces[k]];
     d /= V[c];
@@ -395,7 +449,7 @@ __global__ __launch_bounds__(kTpb) void corrFluxLimitedK(int nF, const label* __
 
 // source -= sum over the cell's faces of (+ffc owned, -ffc neighbour-side), ascending face index
 // (fvm.cuh:293-299, pEqn_cpp.cu:228)
-__global__ __launch_bounds__(kTpb) void corrSourceK(int n, const label* __restrict__ ownerStart,
+__global__ __launch_bounds__(kTpb) void corrSourceK(int n, int nF, const label* __restrict__ ownerStart,
                                                     const label* __restrict__ losortStart,
                                                     const label* __restrict__ losort, const double* __restrict__ ffc,
                                                     double* __restrict__ source)
@@ -403,8 +457,7 @@ __global__ __launch_bounds__(kTpb) void corrSourceK(int n, const label* __restri
     const int c = xcdBlock() * kTpb + threadIdx.x;
     if (c >= n) return;
     double s = 0.0;
-    for (int k = losortStart[c]; k < losortStart[c + 1]; ++k) s -= ffc[losort[k]];
-    for (int f = ownerStart[c]; f < ownerStart[c + 1]; ++f) s += ffc[f];
+    cellFaces(c, nF, ownerStart, losortStart, losort, ffc, ffc, [&](double q, bool owned) { s = owned ? s + q : s - q; });
     source[c] -= s;
 }
 
@@ -423,7 +476,7 @@ void launchDivSource(Ctx& c, const Mesh& m, const double* phi, const double* phi
                      double* source)
 {
     if (!m.nCells) return;
-    divSourceK<<<blocks(m.nCells), kTpb, 0, c.stream>>>(m.nCells, m.ownerStart.p, m.losortStart.p, m.losort.p,
+    divSourceK<<<blocks(m.nCells), kTpb, 0, c.stream>>>(m.nCells, m.nFaces, m.ownerStart.p, m.losortStart.p, m.losort.p,
                                                         m.bndStart.p, m.bndFaces.p, phi, phib, V, sign, source);
     hipCheck(hipGetLastError(), "div source");
 }
@@ -449,7 +502,7 @@ void launchLaplacianCorr(Ctx& c, const Mesh& m, const double* grad, const double
         corrFluxK<<<blocks(m.nFaces), kTpb, 0, c.stream>>>(m.nFaces, m.owner.p, m.neighbour.p, grad, w, corrVec, gammaf,
                                                            magSf, ffc);
     if (source && m.nCells)
-        corrSourceK<<<blocks(m.nCells), kTpb, 0, c.stream>>>(m.nCells, m.ownerStart.p, m.losortStart.p, m.losort.p,
+        corrSourceK<<<blocks(m.nCells), kTpb, 0, c.stream>>>(m.nCells, m.nFaces, m.ownerStart.p, m.losortStart.p, m.losort.p,
                                                              ffc, source);
     hipCheck(hipGetLastError(), "laplacian correction");
 }
@@ -457,7 +510,7 @@ void launchLaplacianCorr(Ctx& c, const Mesh& m, const double* grad, const double
 void launchAmul(Ctx& c, const Mesh& m, const LduView& A, const double* x, double* y)
 {
     if (m.nCells == 0) return;
-    amulK<<<blocks(m.nCells), kTpb, 0, c.stream>>>(m.nCells, m.ownerStart.p, m.losortStart.p, m.losort.p,
+    amulK<<<blocks(m.nCells), kTpb, 0, c.stream>>>(m.nCells, m.nFaces, m.ownerStart.p, m.losortStart.p, m.losort.p,
                                                    m.losortOwner.p, m.neighbour.p, A.diag, A.upper, A.lower, x, y);
     hipCheck(hipGetLastError(), "amul");
 }
@@ -465,7 +518,7 @@ void launchAmul(Ctx& c, const Mesh& m, const LduView& A, const double* x, double
 void launchResidual(Ctx& c, const Mesh& m, const LduView& A, const double* x, const double* b, double* r)
 {
     if (m.nCells == 0) return;
-    residualK<<<blocks(m.nCells), kTpb, 0, c.stream>>>(m.nCells, m.ownerStart.p, m.losortStart.p, m.losort.p,
+    residualK<<<blocks(m.nCells), kTpb, 0, c.stream>>>(m.nCells, m.nFaces, m.ownerStart.p, m.losortStart.p, m.losort.p,
                                                        m.losortOwner.p, m.neighbour.p, A.diag, A.upper, A.lower, x,
                                                        b, r);
     hipCheck(hipGetLastError(), "residual");
@@ -478,7 +531,7 @@ void launchNormFactor(Ctx& c, const Mesh& m, const LduView& A, const double* psi
     if (c.sequentialReduce)
     {
         sumSeqK<<<1, 64, 0, c.stream>>>(n, psi, sumPsi);
-        normFactorSeqK<<<1, 64, 0, c.stream>>>(n, m.ownerStart.p, m.losortStart.p, m.losort.p, m.losortOwner.p,
+        normFactorSeqK<<<1, 64, 0, c.stream>>>(n, m.nFaces, m.ownerStart.p, m.losortStart.p, m.losort.p, m.losortOwner.p,
                                                m.neighbour.p, A.diag, A.upper, A.lower, psi, b, sumPsi, out);
     }
     else
@@ -487,7 +540,7 @@ void launchNormFactor(Ctx& c, const Mesh& m, const LduView& A, const double* psi
         double* pa = c.partials.p + 3 * (size_t)kMaxReduceBlocks;
         sumK<<<g, kReduceBlock, 0, c.stream>>>(n, psi, pa);
         finishK<<<1, kFinishBlock, 0, c.stream>>>(g, pa, StoreTo{sumPsi}, nullptr);
-        normFactorK<<<g, kReduceBlock, 0, c.stream>>>(n, m.ownerStart.p, m.losortStart.p, m.losort.p,
+        normFactorK<<<g, kReduceBlock, 0, c.stream>>>(n, m.nFaces, m.ownerStart.p, m.losortStart.p, m.losort.p,
                                                       m.losortOwner.p, m.neighbour.p, A.diag, A.upper, A.lower, psi,
                                                       b, sumPsi, pa);
         finishK<<<1, kFinishBlock, 0, c.stream>>>(g, pa, NormPost{out}, nullptr);
@@ -502,7 +555,7 @@ void launchLaplacian(Ctx& c, const Mesh& m, const double* dc, const double* gamm
         lapFaceK<<<blocks(m.nFaces), kTpb, 0, c.stream>>>(m.nFaces, dc, gammaf, magSf, upper,
                                                           lower == upper ? nullptr : lower);
     if (m.nCells)
-        lapDiagK<<<blocks(m.nCells), kTpb, 0, c.stream>>>(m.nCells, m.ownerStart.p, m.losortStart.p, m.losort.p,
+        lapDiagK<<<blocks(m.nCells), kTpb, 0, c.stream>>>(m.nCells, m.nFaces, m.ownerStart.p, m.losortStart.p, m.losort.p,
                                                           upper, diag);
     hipCheck(hipGetLastError(), "laplacian");
 }
@@ -519,7 +572,7 @@ void launchDivUpwind(Ctx& c, const Mesh& m, const double* phi, double* diag, dou
 {
     if (m.nFaces) divFaceK<<<blocks(m.nFaces), kTpb, 0, c.stream>>>(m.nFaces, phi, upper, lower);
     if (m.nCells)
-        divDiagK<<<blocks(m.nCells), kTpb, 0, c.stream>>>(m.nCells, m.ownerStart.p, m.losortStart.p, m.losort.p,
+        divDiagK<<<blocks(m.nCells), kTpb, 0, c.stream>>>(m.nCells, m.nFaces, m.ownerStart.p, m.losortStart.p, m.losort.p,
                                                           upper, lower, diag);
     hipCheck(hipGetLastError(), "div upwind");
 }
@@ -529,7 +582,7 @@ void launchDivCentral(Ctx& c, const Mesh& m, const double* phi, const double* we
 {
     if (m.nFaces) divFaceLinearK<<<blocks(m.nFaces), kTpb, 0, c.stream>>>(m.nFaces, phi, weights, upper, lower);
     if (m.nCells)
-        divDiagK<<<blocks(m.nCells), kTpb, 0, c.stream>>>(m.nCells, m.ownerStart.p, m.losortStart.p, m.losort.p,
+        divDiagK<<<blocks(m.nCells), kTpb, 0, c.stream>>>(m.nCells, m.nFaces, m.ownerStart.p, m.losortStart.p, m.losort.p,
                                                           upper, lower, diag);
     hipCheck(hipGetLastError(), "div linear");
 }
