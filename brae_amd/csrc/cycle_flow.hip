@@ -333,7 +333,7 @@ __global__ __launch_bounds__(kThreads) void flowCycleK(const FlowGrid* __restric
     __shared__ int chunksOf[kMaxFlowGrids];
     const int lane = threadIdx.x & 63, quarter = (int)__builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const unsigned tag = launchTag(state);
-    Chunks order(state, slots);
+    GroupChunks order(state, slots);
     if ((int)threadIdx.x < st.T) chunksOf[threadIdx.x] = (grids[threadIdx.x].n + 63) >> 6;
     __syncthreads();
     const int nSteps = st.count(), xs = max(nPre - 1, 0);
@@ -597,7 +597,7 @@ __global__ __launch_bounds__(kThreads) void flowCycleK(const FlowGrid* __restric
             }
         }
     }
-    leave(state, tag, (unsigned)(nPre + nPost + 2));
+    leave(order, (unsigned)first, tag, (unsigned)(nPre + nPost + 2));   // first: the chunks of every step
 }
 
 } // namespace
@@ -659,7 +659,7 @@ void flowCycleBuild(Ctx& c, Amg& a)
     if (a.flowWords.n != wordAt[T] || !a.flowState.n)
     {
         a.flowWords.upload(std::vector<Word>(wordAt[T], 0ull), c.stream);
-        a.flowState.upload(std::vector<unsigned>{0u, 0u, 1u}, c.stream);
+        a.flowState.upload(firstHandState(), c.stream);
     }
     std::vector<FlowGrid> d(T);
     for (int t = 0; t < T; ++t)

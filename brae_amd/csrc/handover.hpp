@@ -6,10 +6,12 @@
 // to be ordered -- no fence, no barrier. Every wait ends: a chunk needs values of earlier chunks only, those
 // were taken earlier, by waves that were running and leave no chunk unfinished; the earliest unfinished chunk
 // never waits. Nothing depends on how many waves run at once. The tags grow with every launch (kept in device
-// memory and advanced by the last wave to leave, so a captured launch replays correctly).
+// memory and advanced by the last workgroup to leave, so a captured launch replays correctly; chunks.hpp).
 #pragma once
 
 #include "mfv_internal.hpp"
+
+#include "chunks.hpp"
 
 namespace mfv {
 
@@ -69,6 +71,9 @@ struct Hand<float>
     }
 };
 
+// the state a launch's first predecessor would have left: tag 1, so that no word as allocated (0) passes for a value
+inline std::vector<unsigned> firstHandState() { return {0u, 0u, 1u, 0u}; }
+
 template <typename T>
 __device__ __forceinline__ T awaitValue(const Word* p, int i, unsigned tag)
 {
@@ -79,57 +84,6 @@ __device__ __forceinline__ T awaitValue(const Word* p, int i, unsigned tag)
         v = Hand<T>::get(p, i);
     }
     return v.value();
-}
-
-// the launch's state in device memory: the next chunk, the workgroups that have left, the tag
-enum : int { kNext = 0, kDone = 1, kTag = 2, kHandState = 3 };
-
-__device__ __forceinline__ unsigned launchTag(const unsigned* state)
-{
-    return __hip_atomic_load(state + kTag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-
-// the next chunk, for a workgroup of one wave
-__device__ __forceinline__ int takeChunk(unsigned* state)
-{
-    unsigned t = 0;
-    if (threadIdx.x == 0) t = __hip_atomic_fetch_add(state + kNext, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    return (int)__builtin_amdgcn_readfirstlane(t);
-}
-
-// A larger workgroup's chunks in order: next() is the one to work on (the same in every thread). A chunk is asked for
-// while the one before it is worked on, which keeps the order's promise: the workgroup finishes that one first.
-struct Chunks
-{
-    unsigned* state;
-    int* slots;      // two, in LDS
-    unsigned ahead;  // thread 0: the chunk asked for
-    int turn;
-    __device__ __forceinline__ Chunks(unsigned* s, int* lds) : state(s), slots(lds), ahead(0), turn(0) { ask(); }
-    __device__ __forceinline__ void ask()
-    {
-        if (threadIdx.x == 0)
-            ahead = __hip_atomic_fetch_add(state + kNext, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    }
-    __device__ __forceinline__ int next()
-    {
-        if (threadIdx.x == 0) slots[turn] = (int)ahead;
-        __syncthreads();
-        const int t = __builtin_amdgcn_readfirstlane(slots[turn]);
-        turn ^= 1;
-        ask();
-        return t;
-    }
-};
-
-// the last workgroup to leave resets the counter and moves the tag on for the next launch (`by` tags were used)
-__device__ __forceinline__ void leave(unsigned* state, unsigned tag, unsigned by)
-{
-    if (threadIdx.x) return;
-    if (__hip_atomic_fetch_add(state + kDone, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1 != gridDim.x) return;
-    __hip_atomic_store(state + kNext, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    __hip_atomic_store(state + kDone, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    __hip_atomic_store(state + kTag, tag + by, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
 } // namespace mfv

@@ -53,7 +53,7 @@ struct SweepPlan
     int gsLag = 0;            // LDS: a step's neighbours lie fewer steps than this from it
     // LDS: coefficients and cell values in the walks' orders
     DBuf<double> aFwd, aBwd, dFwd, aGs, aGsBack, gsIn;
-    // flow: the hand-over buffer and {next chunk, waves done, tag}
+    // flow: the hand-over buffer and the launches' state (chunks.hpp)
     DBuf<Word> hand;
     DBuf<unsigned> state;
 };
@@ -493,7 +493,8 @@ __global__ __launch_bounds__(64) void flowSubstK(PlanView P, const double* __res
     if (stop && *stop) return;
     const unsigned tag = launchTag(state);
     const int lane = threadIdx.x, total = P.nFwd + (Factor ? 0 : P.nBwd);
-    for (int s = takeChunk(state); s < total; s = takeChunk(state))
+    WaveChunks order(state);
+    for (int s = order.next(); s < total; s = order.next())
     {
         const int back = s >= P.nFwd ? 1 : 0;   // uniform
         Lane<W> L;
@@ -536,7 +537,7 @@ __global__ __launch_bounds__(64) void flowSubstK(PlanView P, const double* __res
                 out[L.c] = v;
         }
     }
-    leave(state, tag, 2);
+    leave(order, (unsigned)total, tag, 2);
 }
 
 // One Gauss-Seidel walk: forward (lower neighbours handed over; upper ones read from psi, where their old
@@ -550,7 +551,8 @@ __global__ __launch_bounds__(64) void flowGsK(int nSteps, const int4* __restrict
 {
     const unsigned tag = launchTag(state);
     const int lane = threadIdx.x;
-    for (int t = takeChunk(state); t < nSteps; t = takeChunk(state))
+    WaveChunks order(state);
+    for (int t = order.next(); t < nSteps; t = order.next())
     {
         Lane<W> L;
         laneLoad<W>(steps, t, cell, self, face, pos, L);
@@ -606,7 +608,7 @@ __global__ __launch_bounds__(64) void flowGsK(int nSteps, const int4* __restrict
             Hand<double>::put(hand, own, tag, v);
         }
     }
-    leave(state, tag, 1);
+    leave(order, (unsigned)nSteps, tag, 1);
 }
 
 // ---------------- host ----------------
@@ -764,7 +766,7 @@ bool planBuild(Ctx& c, Mesh& m, SweepPlan* p)
         return true;
     }
     p->hand.upload(std::vector<Word>(2 * (size_t)n, 0ull), c.stream);
-    p->state.upload(std::vector<unsigned>{0u, 0u, 1u}, c.stream);
+    p->state.upload(firstHandState(), c.stream);
     return true;
 }
 
