@@ -47,6 +47,16 @@ void buildLevels(Ctx& c, Mesh& m)
     s->bwdCells.upload(bc, c.stream);
     hipCheck(hipStreamSynchronize(c.stream), "level schedule");
     m.sched = std::move(s);
+    try
+    {
+        sweepPlan(c, m);
+    }
+    catch (...)
+    {
+        m.sweep.reset();
+        m.sched.reset();
+        throw;
+    }
 }
 
 // rD before inversion: diag - sum over lower faces (ascending) of upper^2 / rD[lower neighbour]

@@ -198,7 +198,7 @@ struct Mesh
     int band = 0;              // largest neighbour - owner over the internal faces
     std::vector<label> hOwner, hNeighbour, hBFaceCell;
     std::unique_ptr<LevelSched> sched;   // built on first use by the sequential sweeps (DIC, Gauss-Seidel)
-    std::unique_ptr<SweepPlan, SweepPlanDeleter> sweep;   // on first use by a sweep on the schedule
+    std::unique_ptr<SweepPlan, SweepPlanDeleter> sweep;   // built with it
     std::unique_ptr<BicgWork, BicgWorkDeleter> bicg;   // PBiCGStab's vectors, on first use
 };
 

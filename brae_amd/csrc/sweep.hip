@@ -31,11 +31,12 @@ namespace mfv {
 struct Walk
 {
     int nSteps = 0, nEntries = 0;
-    DBuf<int4> steps;         // {first lane, cells, first entry, entries per cell}
-    DBuf<int> cell, self;     // per lane: the cell; its place, or (Gauss-Seidel) its number of lower faces
-    DBuf<int> face, pos;      // entries
-    DBuf<int> entryCell;      // LDS: the entry's cell
-    DBuf<unsigned> at;        // LDS: in place of pos
+    const int4* steps = nullptr;   // {first lane, cells, first entry, entries per cell}
+    const int* cell = nullptr;     // per lane: the cell (the level schedule's list);
+    int* self = nullptr;           // its place, or (Gauss-Seidel) its number of lower faces
+    int *face = nullptr, *pos = nullptr;   // entries
+    int* entryCell = nullptr;      // LDS: the entry's cell
+    unsigned* at = nullptr;        // LDS: in place of pos
 };
 
 struct SweepPlan
@@ -45,16 +46,18 @@ struct SweepPlan
     bool wide = false;        // a cell with more lower or owned faces than the narrow kernels load ahead
     bool packed = false;      // LDS: the substitution's coefficients are the last factorisation's
     int n = 0, threads = 64;
-    const Ctx* owner = nullptr;   // the buffers below belong to one context's stream
+    DBuf<int4> steps, gsSteps;     // the walks' steps
+    DBuf<uint8_t> mem, gsMem;      // and the rest of them
+    int* place = nullptr;          // per cell
     Walk fwd, bwd;            // lower faces ascending; owned faces descending
     bool gsReady = false, gsUsable = false;
     Walk gs;                  // Gauss-Seidel's forward walk: both runs of faces, ascending
     int gsAhead = 0;          // its entries loaded ahead
     int gsLag = 0;            // LDS: a step's neighbours lie fewer steps than this from it
     // LDS: coefficients and cell values in the walks' orders
-    DBuf<double> aFwd, aBwd, dFwd, aGs, aGsBack, gsIn;
+    double *aFwd = nullptr, *aBwd = nullptr, *dFwd = nullptr, *aGs = nullptr, *aGsBack = nullptr, *gsIn = nullptr;
     // flow: the hand-over buffer and the launches' state (chunks.hpp)
-    DBuf<Word> hand;
+    Word* hand = nullptr;
     DBuf<unsigned> state;
 };
 void SweepPlanDeleter::operator()(SweepPlan* p) const { delete p; }
@@ -67,7 +70,8 @@ constexpr int kLdsCells = 20000;
 constexpr int kLdsThreads = 512;
 // Above this a mesh keeps a launch per level: the gain falls as the levels widen and the values' words (16
 // bytes) become traffic. A DILU solve of n^3 cells against a launch per level: 6.6x at 64^3, 6.0x at 128^3,
-// 3.3x at 200^3, 2.0x at 272^3 (20 M cells, 165 -> 83 ms); the plan takes about 90 bytes a cell.
+// 3.3x at 200^3, 2.0x at 272^3 (20 M cells, 165 -> 83 ms); the plan takes about 76 bytes a cell of a hex mesh, and
+// 52 more with Gauss-Seidel's walk.
 constexpr int kFlowMaxCells = 1 << 25;
 // Entries of a step's cell that are loaded ahead, by the most that a cell of the mesh has (a hex mesh's have
 // three lower and three owned faces, agglomerated ones more); a cell's entries past these are loaded where
@@ -619,95 +623,199 @@ bool capturing(hipStream_t s)
     return hipStreamIsCapturing(s, &st) == hipSuccess && st != hipStreamCaptureStatusNone;
 }
 
-// per cell, its faces as neighbour (ascending) and as owner (a contiguous run)
-struct Runs
+// ---------------- the plan, laid out on the device ----------------
+//
+// The first sweep on a mesh pays for it, so it is made where the addressing is: the steps' widths by a launch, their
+// entries' places added up on the host (16 bytes a step), the entries written by another launch. First calls on a
+// mesh, level schedule and all, against a launch per level without a plan: one DIC application 0.15 ms and 0.3 at
+// 10^3 cells, 2.8 and 5.1 at 64^3, 20 and 24 at 128^3, 212 and 215 at 20 M; two Gauss-Seidel sweeps 0.23 and 0.22,
+// 2.8 and 5.0, 20 and 24, 214 and 218. (By one host thread with uploads 128^3 took 151 and 257, 20 M 1,700 and 3,200.)
+
+// the faces a walk's cells have as entries: the lower ones ascending, the owned ones descending, or both ascending
+enum WalkKind : int { kLowerFaces, kOwnedFaces, kAllFaces };
+
+struct MeshView
 {
-    std::vector<int> ls, lo, os;
-    explicit Runs(const Mesh& m) : ls(m.nCells + 1, 0), lo(m.nFaces), os(m.nCells + 1, 0)
-    {
-        for (int f = 0; f < m.nFaces; ++f)
-        {
-            ++ls[m.hNeighbour[f] + 1];
-            ++os[m.hOwner[f] + 1];
-        }
-        for (int c = 0; c < m.nCells; ++c)
-        {
-            ls[c + 1] += ls[c];
-            os[c + 1] += os[c];
-        }
-        std::vector<int> at(ls.begin(), ls.end() - 1);
-        for (int f = 0; f < m.nFaces; ++f) lo[at[m.hNeighbour[f]]++] = f;
-    }
+    const label* __restrict__ ownerStart;
+    const label* __restrict__ neighbour;
+    const label* __restrict__ losortStart;
+    const label* __restrict__ losort;
+    const label* __restrict__ losortOwner;
 };
+MeshView viewOf(const Mesh& m)
+{
+    return MeshView{m.ownerStart.p, m.neighbour.p, m.losortStart.p, m.losort.p, m.losortOwner.p};
+}
+
+__global__ __launch_bounds__(kTpb) void placeK(int n, const int* __restrict__ order, int* __restrict__ place)
+{
+    const int i = blockIdx.x * kTpb + threadIdx.x;
+    if (i < n) place[order[i]] = i;
+}
+
+__global__ __launch_bounds__(kTpb) void zeroWordsK(size_t n, Word* __restrict__ w)
+{
+    const size_t i = (size_t)blockIdx.x * kTpb + threadIdx.x;
+    if (i < n) w[i] = 0ull;
+}
+
+// a step's widest cell into its w, a wave to a step; the first nA steps are walk A's, the rest walk B's
+__global__ __launch_bounds__(kTpb) void stepWidthK(int nSteps, int nA, MeshView M, WalkKind kindA,
+                                                   const int* __restrict__ orderA, WalkKind kindB,
+                                                   const int* __restrict__ orderB, int4* __restrict__ steps)
+{
+    const int s = blockIdx.x * (kTpb / 64) + (int)(threadIdx.x >> 6), lane = threadIdx.x & 63;
+    if (s >= nSteps) return;
+    const WalkKind kind = s < nA ? kindA : kindB;
+    const int* order = s < nA ? orderA : orderB;
+    const int4 d = steps[s];
+    int k = 0;
+    for (int i = lane; i < d.y; i += 64)
+    {
+        const int q = order[d.x + i];
+        const int nl = M.losortStart[q + 1] - M.losortStart[q], no = M.ownerStart[q + 1] - M.ownerStart[q];
+        k = max(k, kind == kLowerFaces ? nl : kind == kOwnedFaces ? no : nl + no);
+    }
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) k = max(k, __shfl_xor(k, o, 64));
+    if (lane == 0) steps[s].w = k;
+}
+
+// A walk's entries, a wave to a step: every one that its steps have room for, past a cell's faces those that name
+// none. stepOf (may be null): per cell, its step.
+template <WalkKind Kind, bool Lds>
+__global__ __launch_bounds__(kTpb) void entriesK(int n, Walk W, MeshView M, const int* __restrict__ place,
+                                                 int* __restrict__ stepOf)
+{
+    const int s = blockIdx.x * (kTpb / 64) + (int)(threadIdx.x >> 6), lane = threadIdx.x & 63;
+    if (s >= W.nSteps) return;
+    const int4 d = W.steps[s];
+    for (int i = lane; i < d.y; i += 64)
+    {
+        const int q = W.cell[d.x + i];
+        const int l0 = M.losortStart[q], nl = Kind == kOwnedFaces ? 0 : M.losortStart[q + 1] - l0;
+        const int o0 = M.ownerStart[q], no = Kind == kLowerFaces ? 0 : M.ownerStart[q + 1] - o0;
+        W.self[d.x + i] = Kind == kAllFaces ? nl : place[q];
+        if (stepOf) stepOf[q] = s;
+        for (int k = 0; k < d.w; ++k)
+        {
+            const size_t e = Lds ? (size_t)d.z + (size_t)(k & ~1) * d.y + 2 * i + (k & 1) : (size_t)d.z + (size_t)k * d.y + i;
+            int f = -1, p = Lds ? n : 0;
+            if (k < nl)
+            {
+                f = M.losort[l0 + k];
+                p = place[M.losortOwner[l0 + k]];
+            }
+            else if (k < nl + no)
+            {
+                f = Kind == kOwnedFaces ? o0 + no - 1 - k : o0 + k - nl;
+                const int c = M.neighbour[f];
+                // Gauss-Seidel reads an upper neighbour's old value, in memory by cell
+                p = Kind == kAllFaces && !Lds ? c : place[c];
+            }
+            W.face[e] = f;
+            if (Lds)
+            {
+                W.entryCell[e] = f >= 0 ? q : 0;
+                W.at[e] = 8u * (unsigned)p;
+            }
+            else
+                W.pos[e] = p;
+        }
+    }
+}
+
+// the most steps that lie between a face's two cells
+__global__ __launch_bounds__(kTpb) void stepReachK(int nF, const label* __restrict__ owner,
+                                                   const label* __restrict__ neighbour,
+                                                   const int* __restrict__ stepOf, int* __restrict__ reach)
+{
+    const int f = blockIdx.x * kTpb + threadIdx.x;
+    if (f < nF) atomicMax(reach, abs(stepOf[neighbour[f]] - stepOf[owner[f]]));
+}
+
+inline int blocks(int n) { return (n + kTpb - 1) / kTpb; }
+inline int waveBlocks(int n) { return (n + kTpb / 64 - 1) / (kTpb / 64); }
 
 // Room for a plan's entries: a hex mesh fills about one per face and run, an agglomerated grid two or three.
 // A cell with very many faces in a wide level would pad its whole step; such a mesh keeps a launch per level.
 long long entryRoom(const Mesh& m) { return std::min(0x7fffffffLL, 16LL * ((long long)m.nCells + m.nFaces)); }
 
-// One walk: `order` cut at the levels' starts into steps of at most `threads` cells, each with room for its
-// widest cell's entries and for at least `least`. count(q): cell q's entries; list(q, put): put(face, place
-// or cell) for each in order; self(q) what the lanes carry. False where it would not fit.
-template <typename Count, typename List, typename Self>
-bool buildWalk(Ctx& c, Walk& w, const std::vector<int>& start, const std::vector<int>& order, bool lds, int threads,
-               int least, long long room, Count count, List list, Self self)
+// `steps` gets the levels cut into steps of at most `threads` cells
+void cutSteps(const std::vector<int>& start, int threads, std::vector<int4>& steps)
 {
-    std::vector<int4> steps;
-    long long entries = 0;
     for (size_t l = 0; l + 1 < start.size(); ++l)
-        for (int a = start[l]; a < start[l + 1]; a += threads)
-        {
-            const int cnt = std::min(threads, start[l + 1] - a);
-            int k = least;
-            for (int i = a; i < a + cnt; ++i) k = std::max(k, count(order[i]));
-            if (lds) k = (k + 1) & ~1;
-            steps.push_back(int4{a, cnt, (int)entries, k});
-            entries += (long long)k * cnt;
-            if (entries > room) return false;
-        }
-    const size_t n = order.size();
-    std::vector<int> sf(n), face(entries, -1), pos(lds ? 0 : entries, 0), own(lds ? entries : 0, 0);
-    std::vector<unsigned> at(lds ? entries : 0, 8u * (unsigned)n);
-    for (const int4& d : steps)
-        for (int i = 0; i < d.y; ++i)
-        {
-            const int q = order[d.x + i];
-            sf[d.x + i] = self(q);
-            int k = 0;
-            list(q, [&](int f, int p) {
-                const size_t e = lds ? (size_t)d.z + (size_t)(k & ~1) * d.y + 2 * i + (k & 1)
-                                     : (size_t)d.z + (size_t)k * d.y + i;
-                ++k;
-                face[e] = f;
-                if (lds)
-                {
-                    own[e] = q;
-                    at[e] = 8u * (unsigned)p;
-                }
-                else
-                    pos[e] = p;
-            });
-        }
-    w.nSteps = (int)steps.size();
-    w.nEntries = (int)entries;
-    w.steps.upload(steps, c.stream);
-    w.cell.upload(order, c.stream);
-    w.self.upload(sf, c.stream);
-    w.face.upload(face, c.stream);
-    if (lds)
+        for (int a = start[l]; a < start[l + 1]; a += threads) steps.push_back(int4{a, std::min(threads, start[l + 1] - a), 0, 0});
+}
+
+int widestCell(const std::vector<int4>& steps)
+{
+    int most = 0;
+    for (const int4& d : steps) most = std::max(most, d.w);
+    return most;
+}
+
+// Room for a walk's steps [a, b): the entries of each from its widest cell's, and at least `least`. False where they
+// would not fit.
+bool placeEntries(std::vector<int4>& steps, size_t a, size_t b, bool lds, int least, long long room, Walk& w)
+{
+    long long entries = 0;
+    for (size_t s = a; s < b; ++s)
     {
-        w.entryCell.upload(own, c.stream);
-        w.at.upload(at, c.stream);
+        int k = std::max(least, steps[s].w);
+        if (lds) k = (k + 1) & ~1;
+        steps[s].z = (int)entries;
+        steps[s].w = k;
+        entries += (long long)k * steps[s].y;
+        if (entries > room) return false;
     }
-    else
-        w.pos.upload(pos, c.stream);
+    w.nSteps = (int)(b - a);
+    w.nEntries = (int)entries;
     return true;
 }
 
-std::vector<int> placesOf(const std::vector<int>& fwd)
+// arrays in one allocation: first with the base null, for the bytes, then with it
+struct Carve
 {
-    std::vector<int> place(fwd.size());
-    for (size_t i = 0; i < fwd.size(); ++i) place[fwd[i]] = (int)i;
-    return place;
+    uint8_t* base;
+    size_t used = 0;
+    template <typename T>
+    void operator()(T*& p, size_t n)
+    {
+        p = reinterpret_cast<T*>(base + used);
+        used += (n * sizeof(T) + 255) / 256 * 256;
+    }
+};
+template <typename Fn>
+void carve(DBuf<uint8_t>& mem, Fn fn)
+{
+    Carve size{nullptr};
+    fn(size);
+    mem.resize(size.used);
+    Carve at{mem.p};
+    fn(at);
+}
+void carveWalk(Carve& c, Walk& w, int n, bool lds)
+{
+    c(w.self, (size_t)n);
+    c(w.face, (size_t)w.nEntries);
+    if (lds)
+    {
+        c(w.entryCell, (size_t)w.nEntries);
+        c(w.at, (size_t)w.nEntries);
+    }
+    else
+        c(w.pos, (size_t)w.nEntries);
+}
+
+template <WalkKind Kind>
+void writeEntries(Ctx& c, const Mesh& m, const SweepPlan& p, const Walk& w, int* stepOf = nullptr)
+{
+    if (p.lds)
+        entriesK<Kind, true><<<waveBlocks(w.nSteps), kTpb, 0, c.stream>>>(p.n, w, viewOf(m), p.place, stepOf);
+    else
+        entriesK<Kind, false><<<waveBlocks(w.nSteps), kTpb, 0, c.stream>>>(p.n, w, viewOf(m), p.place, stepOf);
+    hipCheck(hipGetLastError(), "sweep plan");
 }
 
 // whether the plan's arrays fit the device; without room the mesh keeps a launch per level
@@ -731,108 +839,113 @@ bool planBuild(Ctx& c, Mesh& m, SweepPlan* p)
     const LevelSched& S = *m.sched;
     const int n = m.nCells;
     p->n = n;
-    p->owner = &c;
     p->lds = n <= kLdsCells;
-    int widest = 1, most = 0;
+    int widest = 1;
     for (const std::vector<int>* st : {&S.fwdStart, &S.bwdStart})
         for (size_t l = 0; l + 1 < st->size(); ++l) widest = std::max(widest, (*st)[l + 1] - (*st)[l]);
     p->threads = p->lds ? std::min(kLdsThreads, (widest + 63) / 64 * 64) : 64;
-    const std::vector<int> fwd = S.fwdCells.download(c.stream), bwd = S.bwdCells.download(c.stream);
-    const std::vector<int> place = placesOf(fwd);
-    const Runs R(m);
-    for (int q = 0; q < n; ++q) most = std::max(most, std::max(R.ls[q + 1] - R.ls[q], R.os[q + 1] - R.os[q]));
+    std::vector<int4> steps;
+    cutSteps(S.fwdStart, p->threads, steps);
+    const size_t nF = steps.size();
+    cutSteps(S.bwdStart, p->threads, steps);
+    p->steps.upload(steps, c.stream);
+    stepWidthK<<<waveBlocks((int)steps.size()), kTpb, 0, c.stream>>>((int)steps.size(), (int)nF, viewOf(m), kLowerFaces,
+                                                                      S.fwdCells.p, kOwnedFaces, S.bwdCells.p, p->steps.p);
+    hipCheck(hipGetLastError(), "sweep plan");
+    steps = p->steps.download(c.stream);
     const int narrow = p->lds ? kLdsNarrow : kFlowNarrow;
-    p->wide = most > narrow;
+    p->wide = widestCell(steps) > narrow;
     const int least = p->wide ? kWide : narrow;
-    const auto at = [&](int q) { return place[q]; };
-    if (!buildWalk(c, p->fwd, S.fwdStart, fwd, p->lds, p->threads, least, entryRoom(m),
-                   [&](int q) { return R.ls[q + 1] - R.ls[q]; },
-                   [&](int q, auto put) {
-                       for (int k = R.ls[q]; k < R.ls[q + 1]; ++k) put(R.lo[k], place[m.hOwner[R.lo[k]]]);
-                   },
-                   at) ||
-        !buildWalk(c, p->bwd, S.bwdStart, bwd, p->lds, p->threads, least, entryRoom(m),
-                   [&](int q) { return R.os[q + 1] - R.os[q]; },
-                   [&](int q, auto put) {
-                       for (int f = R.os[q + 1] - 1; f >= R.os[q]; --f) put(f, place[m.hNeighbour[f]]);
-                   },
-                   at))
+    if (!placeEntries(steps, 0, nF, p->lds, least, entryRoom(m), p->fwd) ||
+        !placeEntries(steps, nF, steps.size(), p->lds, least, entryRoom(m), p->bwd))
         return false;
-    if (p->lds)
-    {
-        p->aFwd.resize(p->fwd.nEntries);
-        p->aBwd.resize(p->bwd.nEntries);
-        p->dFwd.resize(n);
-        return true;
-    }
-    p->hand.upload(std::vector<Word>(2 * (size_t)n, 0ull), c.stream);
+    p->steps.upload(steps, c.stream);
+    p->fwd.steps = p->steps.p;
+    p->bwd.steps = p->steps.p + nF;
+    p->fwd.cell = S.fwdCells.p;
+    p->bwd.cell = S.bwdCells.p;
+    carve(p->mem, [&](Carve& at) {
+        at(p->place, (size_t)n);
+        carveWalk(at, p->fwd, n, p->lds);
+        carveWalk(at, p->bwd, n, p->lds);
+        if (p->lds)
+        {
+            at(p->aFwd, (size_t)p->fwd.nEntries);
+            at(p->aBwd, (size_t)p->bwd.nEntries);
+            at(p->dFwd, (size_t)n);
+        }
+        else
+            at(p->hand, 2 * (size_t)n);
+    });
+    placeK<<<blocks(n), kTpb, 0, c.stream>>>(n, S.fwdCells.p, p->place);
+    writeEntries<kLowerFaces>(c, m, *p, p->fwd);
+    writeEntries<kOwnedFaces>(c, m, *p, p->bwd);
+    if (p->lds) return true;
+    zeroWordsK<<<blocks(2 * n), kTpb, 0, c.stream>>>(2 * (size_t)n, p->hand);
+    hipCheck(hipGetLastError(), "sweep plan");
     p->state.upload(firstHandState(), c.stream);
     return true;
 }
 
-// The mesh's plan, built on first use, or null: a mesh without faces or above kFlowMaxCells, a plan that
-// cannot be uploaded in a capture or would not fit, or one whose buffers another context is using.
-SweepPlan* planOf(Ctx& c, Mesh& m)
-{
-    if (!m.sched || !m.nFaces || m.nCells > kFlowMaxCells) return nullptr;
-    if (m.sweep) return m.sweep->usable && m.sweep->owner == &c ? m.sweep.get() : nullptr;
-    if (capturing(c.stream)) return nullptr;
-    std::unique_ptr<SweepPlan, SweepPlanDeleter> p(new SweepPlan());
-    if (!fits([&] { return planBuild(c, m, p.get()); })) p.reset(new SweepPlan());   // not usable
-    else p->usable = true;
-    m.sweep = std::move(p);
-    return m.sweep->usable ? m.sweep.get() : nullptr;
-}
+// the mesh's plan, or null: a mesh without faces or above kFlowMaxCells, or a plan that would not fit
+SweepPlan* planOf(const Mesh& m) { return m.sweep && m.sweep->usable ? m.sweep.get() : nullptr; }
 
-// the forward walk of Gauss-Seidel (both runs of a cell's faces); an upper neighbour's old value is found in
-// LDS by place, in memory by cell
+// the forward walk of Gauss-Seidel (both runs of a cell's faces), on the first such sweep outside a capture
 bool planGs(Ctx& c, Mesh& m, SweepPlan& p)
 {
     if (p.gsReady) return p.gsUsable;
     if (capturing(c.stream)) return false;
     const LevelSched& S = *m.sched;
-    const std::vector<int> fwd = S.fwdCells.download(c.stream);
-    const std::vector<int> place = placesOf(fwd);
-    const Runs R(m);
-    int most = 0;
-    for (int q = 0; q < m.nCells; ++q) most = std::max(most, R.ls[q + 1] - R.ls[q] + R.os[q + 1] - R.os[q]);
-    p.gsAhead = most <= kGsNarrow ? kGsNarrow : most <= kGsMiddle ? kGsMiddle : kGsWide;
     p.gsReady = true;
     p.gsUsable = fits([&] {
-        if (!buildWalk(c, p.gs, S.fwdStart, fwd, p.lds, p.threads, p.gsAhead, entryRoom(m),
-                       [&](int q) { return R.ls[q + 1] - R.ls[q] + R.os[q + 1] - R.os[q]; },
-                       [&](int q, auto put) {
-                           for (int k = R.ls[q]; k < R.ls[q + 1]; ++k) put(R.lo[k], place[m.hOwner[R.lo[k]]]);
-                           for (int f = R.os[q]; f < R.os[q + 1]; ++f)
-                               put(f, p.lds ? place[m.hNeighbour[f]] : m.hNeighbour[f]);
-                       },
-                       [&](int q) { return R.ls[q + 1] - R.ls[q]; }))
-            return false;
+        std::vector<int4> steps;
+        cutSteps(S.fwdStart, p.threads, steps);
+        p.gsSteps.upload(steps, c.stream);
+        const int nS = (int)steps.size();
+        stepWidthK<<<waveBlocks(nS), kTpb, 0, c.stream>>>(nS, nS, viewOf(m), kAllFaces, S.fwdCells.p, kAllFaces, S.fwdCells.p,
+                                                          p.gsSteps.p);
+        hipCheck(hipGetLastError(), "sweep plan");
+        steps = p.gsSteps.download(c.stream);
+        const int most = widestCell(steps);
+        p.gsAhead = most <= kGsNarrow ? kGsNarrow : most <= kGsMiddle ? kGsMiddle : kGsWide;
+        if (!placeEntries(steps, 0, steps.size(), p.lds, p.gsAhead, entryRoom(m), p.gs)) return false;
+        p.gsSteps.upload(steps, c.stream);
+        p.gs.steps = p.gsSteps.p;
+        p.gs.cell = S.fwdCells.p;
+        int *stepOf = nullptr, *reach = nullptr;
+        carve(p.gsMem, [&](Carve& at) {
+            carveWalk(at, p.gs, p.n, p.lds);
+            if (!p.lds) return;
+            at(p.aGs, (size_t)p.gs.nEntries);
+            at(p.aGsBack, (size_t)p.bwd.nEntries);
+            at(p.gsIn, 4 * (size_t)p.n);
+            at(stepOf, (size_t)p.n);
+            at(reach, 2);
+        });
+        writeEntries<kAllFaces>(c, m, p, p.gs, stepOf);
         if (!p.lds) return true;
-        std::vector<int> stepOf(p.n);
-        const std::vector<int4> steps = p.gs.steps.download(c.stream);
-        for (int t = 0; t < (int)steps.size(); ++t)
-            for (int i = 0; i < steps[t].y; ++i) stepOf[fwd[steps[t].x + i]] = t;
-        p.gsLag = 1;
-        for (int f = 0; f < m.nFaces; ++f)
-            p.gsLag = std::max(p.gsLag, 1 + std::abs(stepOf[m.hNeighbour[f]] - stepOf[m.hOwner[f]]));
-        p.aGs.resize(p.gs.nEntries);
-        p.aGsBack.resize(p.bwd.nEntries);
-        p.gsIn.resize(4 * (size_t)p.n);
+        int r = 0;
+        zeroWordsK<<<1, kTpb, 0, c.stream>>>(1, reinterpret_cast<Word*>(reach));
+        stepReachK<<<blocks(m.nFaces), kTpb, 0, c.stream>>>(m.nFaces, m.owner.p, m.neighbour.p, stepOf, reach);
+        hipCheck(hipGetLastError(), "sweep plan");
+        hipCheck(hipMemcpyAsync(&r, reach, sizeof(int), hipMemcpyDeviceToHost, c.stream), "sweep plan");
+        hipCheck(hipStreamSynchronize(c.stream), "sweep plan");
+        p.gsLag = r + 1;
         return true;
     });
+    if (!p.gsUsable) p.gsMem.release();
     return p.gsUsable;
 }
 
 PlanView flowView(const SweepPlan& p)
 {
-    return PlanView{p.fwd.nSteps, p.bwd.nSteps, {p.fwd.steps.p, p.bwd.steps.p}, {p.fwd.cell.p, p.bwd.cell.p},
-                    {p.fwd.self.p, p.bwd.self.p}, {p.fwd.face.p, p.bwd.face.p}, {p.fwd.pos.p, p.bwd.pos.p}};
+    return PlanView{p.fwd.nSteps, p.bwd.nSteps, {p.fwd.steps, p.bwd.steps}, {p.fwd.cell, p.bwd.cell},
+                    {p.fwd.self, p.bwd.self}, {p.fwd.face, p.bwd.face}, {p.fwd.pos, p.bwd.pos}};
 }
 
 LdsWalk ldsView(const Walk& w, const double* a)
 {
-    return LdsWalk{w.nSteps, 0, w.steps.p, w.cell.p, w.self.p, w.at.p, a};
+    return LdsWalk{w.nSteps, 0, w.steps, w.cell, w.self, w.at, a};
 }
 
 // Dynamic LDS beyond the default is opted into per kernel; a refusal leaves the launch-per-level path. The
@@ -850,8 +963,6 @@ bool ldsAllowed(K* kernel, size_t bytes)
 
 size_t ldsBytes(const SweepPlan& p) { return sizeof(double) * ((size_t)p.n + 1); }
 
-inline int blocks(int n) { return (n + kTpb - 1) / kTpb; }
-
 // waves of a flow launch, the window of chunks in work: more only poll (64^3: 256 waves 3.87 ms a solve, 1024
 // 4.21, 2048 5.22; 200^3: 34.4, 35.1, 36.6)
 constexpr int kFlowWaves = 256;
@@ -863,11 +974,11 @@ bool factorLds(Ctx& c, SweepPlan& p, const double* diag, const double* upper, co
     p.packed = ldsAllowed(&ldsFactorK<W>, bytes) && ldsAllowed(&ldsSubstK<W>, bytes);
     if (!p.packed) return false;
     const int nF = p.fwd.nEntries, nB = p.bwd.nEntries;
-    packFactorK<<<blocks(std::max(nF, p.n)), kTpb, 0, c.stream>>>(nF, p.fwd.face.p, p.n, p.fwd.cell.p, diag, upper, lower,
-                                                                 p.aFwd.p, p.dFwd.p);
-    ldsFactorK<W><<<1, p.threads, bytes, c.stream>>>(p.n, ldsView(p.fwd, p.aFwd.p), p.dFwd.p, rD);
-    packSubstK<<<blocks(std::max(nF, nB)), kTpb, 0, c.stream>>>(nF, p.fwd.face.p, p.fwd.entryCell.p, nB, p.bwd.face.p,
-                                                               p.bwd.entryCell.p, rD, upper, lower, p.aFwd.p, p.aBwd.p);
+    packFactorK<<<blocks(std::max(nF, p.n)), kTpb, 0, c.stream>>>(nF, p.fwd.face, p.n, p.fwd.cell, diag, upper, lower,
+                                                                 p.aFwd, p.dFwd);
+    ldsFactorK<W><<<1, p.threads, bytes, c.stream>>>(p.n, ldsView(p.fwd, p.aFwd), p.dFwd, rD);
+    packSubstK<<<blocks(std::max(nF, nB)), kTpb, 0, c.stream>>>(nF, p.fwd.face, p.fwd.entryCell, nB, p.bwd.face,
+                                                               p.bwd.entryCell, rD, upper, lower, p.aFwd, p.aBwd);
     return true;
 }
 
@@ -875,7 +986,7 @@ template <int W>
 bool substLds(Ctx& c, SweepPlan& p, const double* r, double* y, const int* stop)
 {
     if (!p.packed) return false;
-    ldsSubstK<W><<<1, p.threads, ldsBytes(p), c.stream>>>(p.n, ldsView(p.fwd, p.aFwd.p), ldsView(p.bwd, p.aBwd.p), p.dFwd.p,
+    ldsSubstK<W><<<1, p.threads, ldsBytes(p), c.stream>>>(p.n, ldsView(p.fwd, p.aFwd), ldsView(p.bwd, p.aBwd), p.dFwd,
                                                          r, y, stop);
     return true;
 }
@@ -886,7 +997,7 @@ void substFlow(Ctx& c, SweepPlan& p, const double* diag, const double* upper, co
 {
     const int steps = p.fwd.nSteps + (Factor ? 0 : p.bwd.nSteps);
     flowSubstK<W, Factor><<<std::min(steps, kFlowWaves), 64, 0, c.stream>>>(flowView(p), diag, upper, lower, rD, r, out,
-                                                                           p.hand.p, p.state.p, stop);
+                                                                           p.hand, p.state.p, stop);
 }
 
 template <int W, int WB>
@@ -897,14 +1008,14 @@ bool gsLds(Ctx& c, SweepPlan& p, const double* diag, const double* upper, const 
     if (!(sym ? ldsAllowed(&ldsGsK<W, WB, true>, bytes) : ldsAllowed(&ldsGsK<W, WB, false>, bytes))) return false;
     const int nF = p.gs.nEntries, nB = sym ? p.bwd.nEntries : 0;
     packGsK<<<blocks(std::max(std::max(nF, nB), p.n)), kTpb, 0, c.stream>>>(
-        nF, p.gs.face.p, nB, p.bwd.face.p, p.n, p.gs.cell.p, diag, upper, b, psi, p.aGs.p, p.aGsBack.p, p.gsIn.p);
-    const LdsWalk F = ldsView(p.gs, p.aGs.p), B = ldsView(p.bwd, p.aGsBack.p);
+        nF, p.gs.face, nB, p.bwd.face, p.n, p.gs.cell, diag, upper, b, psi, p.aGs, p.aGsBack, p.gsIn);
+    const LdsWalk F = ldsView(p.gs, p.aGs), B = ldsView(p.bwd, p.aGsBack);
     // as many teams as the workgroup's room holds, where they gain anything
     const int teams = sym || p.gsLag >= p.gs.nSteps ? 1 : std::max(1, std::min(nSweeps, kLdsThreads / p.threads));
     if (sym)
-        ldsGsK<W, WB, true><<<1, p.threads, bytes, c.stream>>>(p.n, F, B, p.gsIn.p, psi, nSweeps, p.threads, p.gsLag);
+        ldsGsK<W, WB, true><<<1, p.threads, bytes, c.stream>>>(p.n, F, B, p.gsIn, psi, nSweeps, p.threads, p.gsLag);
     else
-        ldsGsK<W, WB, false><<<1, teams * p.threads, bytes, c.stream>>>(p.n, F, B, p.gsIn.p, psi, nSweeps, p.threads,
+        ldsGsK<W, WB, false><<<1, teams * p.threads, bytes, c.stream>>>(p.n, F, B, p.gsIn, psi, nSweeps, p.threads,
                                                                         p.gsLag);
     return true;
 }
@@ -913,16 +1024,26 @@ template <int W, bool Back>
 void gsFlow(Ctx& c, SweepPlan& p, const Walk& w, const double* diag, const double* upper, const double* b, double* psi,
             double* bPrime)
 {
-    flowGsK<W, Back><<<std::min(w.nSteps, kFlowWaves), 64, 0, c.stream>>>(w.nSteps, w.steps.p, w.cell.p, w.self.p, w.face.p,
-                                                                        w.pos.p, diag, upper, b, psi, bPrime, p.hand.p,
+    flowGsK<W, Back><<<std::min(w.nSteps, kFlowWaves), 64, 0, c.stream>>>(w.nSteps, w.steps, w.cell, w.self, w.face, w.pos,
+                                                                        diag, upper, b, psi, bPrime, p.hand,
                                                                         p.state.p);
 }
 
 } // namespace
 
+void sweepPlan(Ctx& c, Mesh& m)
+{
+    m.sweep.reset(new SweepPlan());
+    if (!m.nFaces || m.nCells > kFlowMaxCells) return;
+    if (fits([&] { return planBuild(c, m, m.sweep.get()); }))
+        m.sweep->usable = true;
+    else
+        m.sweep.reset(new SweepPlan());
+}
+
 bool sweepFactor(Ctx& c, Mesh& m, const double* diag, const double* upper, const double* lower, double* rD)
 {
-    SweepPlan* p = planOf(c, m);
+    SweepPlan* p = planOf(m);
     if (!p) return false;
     bool done = true;
     if (p->lds)
@@ -938,7 +1059,7 @@ bool sweepFactor(Ctx& c, Mesh& m, const double* diag, const double* upper, const
 bool sweepSubstitute(Ctx& c, Mesh& m, const double* rD, const double* upper, const double* lower, const double* r,
                      double* y, const int* stop)
 {
-    SweepPlan* p = planOf(c, m);
+    SweepPlan* p = planOf(m);
     if (!p) return false;
     bool done = true;
     if (p->lds)
@@ -954,7 +1075,7 @@ bool sweepSubstitute(Ctx& c, Mesh& m, const double* rD, const double* upper, con
 bool sweepGaussSeidel(Ctx& c, Mesh& m, const double* diag, const double* upper, const double* b, double* psi,
                       int nSweeps, double* bPrime)
 {
-    SweepPlan* p = planOf(c, m);
+    SweepPlan* p = planOf(m);
     if (!p || nSweeps <= 0 || !planGs(c, m, *p)) return false;
     bool done = true;
     if (p->lds)

@@ -1,7 +1,7 @@
 // The sequential sweeps in one launch each (sweep.hip): DIC's and DILU's factorisation, their forward and
-// backward substitution, and Gauss-Seidel, on plans built once per mesh from its level schedule. Each
-// function returns false, having done nothing, where the sweep belongs to the caller's launch-per-level
-// path: a mesh above kFlowMaxCells, one another context sweeps, or a plan that cannot be built now. A
+// backward substitution, and Gauss-Seidel, on a plan built with the mesh's level schedule. Each sweep returns
+// false, having done nothing, where it belongs to the caller's launch-per-level path: a mesh above kFlowMaxCells,
+// a plan that does not fit, or a first Gauss-Seidel inside a capture (its walk is laid out by the first one). A
 // substitution goes with the last factorisation on its mesh: on small meshes that one lays the products
 // rD*lower and rD*upper out in the order the substitution reads them.
 #pragma once
@@ -9,6 +9,9 @@
 #include "mfv_internal.hpp"
 
 namespace mfv {
+
+// lays the mesh's plan out, after its level schedule
+void sweepPlan(Ctx& c, Mesh& m);
 
 // rD = 1/d, d = diag - sum over lower faces (ascending) of upper*lower/d[lower neighbour]
 bool sweepFactor(Ctx& c, Mesh& m, const double* diag, const double* upper, const double* lower, double* rD);

@@ -427,7 +427,9 @@ typedef struct
 int mfv_amg_pcg_solve_batch(mfv_ctx ctx, int n, const mfv_batch_solve* solves, mfv_perf* perfs);
 
 /* ---------------------------------------------------------------------------------------------
- * OpenFOAM's sequential sweeps, level-scheduled on the device and equal to the host loops to the bit.
+ * OpenFOAM's sequential sweeps, level-scheduled on the device and equal to the host loops to the bit. The first
+ * sweep on a mesh builds its level schedule and plan (2 ms for 64^3 cells, 18 for 128^3, 0.2 s for 20 M; about 76
+ * bytes of device memory a cell, 52 more with Gauss-Seidel), which the mesh keeps.
  * ------------------------------------------------------------------------------------------- */
 /* DICPreconditioner: rD (calcReciprocalD) then w = forward/backward substitution of r
  * (src/matrices/lduMatrix/solvers/GAMG/gamg_solver_cpp.cu:194-231; pcg.cu:6-149); synchronises */
