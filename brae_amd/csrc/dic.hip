@@ -260,9 +260,10 @@ __global__ void dicResK(double* st, int* fl)
     fl[G_STOP] = ((it < fl[G_MAXIT] && !conv) || it < fl[G_MINIT]) ? 0 : 1;
 }
 
-void dicApply(Ctx& c, Mesh& m, const LduView& A, const double* rD, const double* r, double* w, const int* stop)
+void dicApply(Ctx& c, Mesh& m, const LduView& A, SweepFactor factor, const double* rD, const double* r, double* w,
+              const int* stop)
 {
-    if (sweepSubstitute(c, m, rD, A.upper, A.upper, r, w, stop)) return;
+    if (sweepSubstitute(c, m, factor, rD, A.upper, A.upper, r, w, stop)) return;
     const LevelSched& s = *m.sched;
     for (size_t l = 0; l + 1 < s.fwdStart.size(); ++l)
     {
@@ -278,9 +279,9 @@ void dicApply(Ctx& c, Mesh& m, const LduView& A, const double* rD, const double*
     }
 }
 
-void dicFactor(Ctx& c, Mesh& m, const LduView& A, double* rD, const int* stop)
+SweepFactor dicFactor(Ctx& c, Mesh& m, const LduView& A, double* rD, const int* stop)
 {
-    if (sweepFactor(c, m, A.diag, A.upper, A.upper, rD)) return;
+    if (const SweepFactor factor = sweepFactor(c, m, A.diag, A.upper, A.upper, rD)) return factor;
     const LevelSched& s = *m.sched;
     for (size_t l = 0; l + 1 < s.fwdStart.size(); ++l)
     {
@@ -289,6 +290,7 @@ void dicFactor(Ctx& c, Mesh& m, const LduView& A, double* rD, const int* stop)
                                                        m.losortOwner.p, A.diag, A.upper, rD);
     }
     invertK<<<blocks(m.nCells), kTpb, 0, c.stream>>>(m.nCells, rD, stop);
+    return 0;
 }
 
 } // namespace
@@ -300,8 +302,8 @@ void launchDicPrecondition(Ctx& c, Mesh& m, const LduView& A, const double* r, d
     if (A.lower != A.upper) throw Error(kErrUnsupported, "mfv: DIC needs a symmetric matrix (lower == upper)");
     if (!m.nCells) return;
     buildLevels(c, m);
-    dicFactor(c, m, A, rD, nullptr);
-    dicApply(c, m, A, rD, r, w, nullptr);
+    const SweepFactor factor = dicFactor(c, m, A, rD, nullptr);
+    dicApply(c, m, A, factor, rD, r, w, nullptr);
     hipCheck(hipGetLastError(), "dic");
 }
 
@@ -332,17 +334,18 @@ void launchGaussSeidel(Ctx& c, Mesh& m, const LduView& A, const double* b, doubl
     hipCheck(hipGetLastError(), "gauss-seidel");
 }
 
-void launchDicFactor(Ctx& c, Mesh& m, const LduView& A, double* rD)
+unsigned launchDicFactor(Ctx& c, Mesh& m, const LduView& A, double* rD)
 {
     if (A.lower != A.upper) throw Error(kErrUnsupported, "mfv: DIC needs a symmetric matrix (lower == upper)");
-    if (!m.nCells) return;
+    if (!m.nCells) return 0;
     buildLevels(c, m);
-    dicFactor(c, m, A, rD, nullptr);
+    const SweepFactor factor = dicFactor(c, m, A, rD, nullptr);
     hipCheck(hipGetLastError(), "dic factor");
+    return factor;
 }
 
-void launchDicSmooth(Ctx& c, Mesh& m, const LduView& A, const double* rD, const double* b, double* psi, int nSweeps,
-                     double* rA, double* w)
+void launchDicSmooth(Ctx& c, Mesh& m, const LduView& A, unsigned factor, const double* rD, const double* b, double* psi,
+                     int nSweeps, double* rA, double* w)
 {
     if (A.lower != A.upper) throw Error(kErrUnsupported, "mfv: the DIC smoother needs a symmetric matrix");
     if (!m.nCells) return;
@@ -350,7 +353,7 @@ void launchDicSmooth(Ctx& c, Mesh& m, const LduView& A, const double* rD, const 
     for (int sw = 0; sw < nSweeps; ++sw)
     {
         launchResidual(c, m, A, psi, b, rA);
-        dicApply(c, m, A, rD, rA, w, nullptr);
+        dicApply(c, m, A, factor, rD, rA, w, nullptr);
         addToK<<<blocks(m.nCells), kTpb, 0, c.stream>>>(m.nCells, w, psi);
     }
     hipCheck(hipGetLastError(), "dic smoother");
@@ -375,11 +378,11 @@ PcgPerf pcgDicSolve(Ctx& c, Mesh& m, const LduView& A, const double* b, double* 
     if (!normFactor) launchNormFactor(c, m, A, psi, b, S + D_NF);
     launchSumMag(c, n, r.p, S + D_T2, 0);
     dicInitK<<<1, 1, 0, c.stream>>>(S, F);
-    dicFactor(c, m, A, rD.p, nullptr);
+    const SweepFactor factor = dicFactor(c, m, A, rD.p, nullptr);
     hipCheck(hipGetLastError(), "pcg-dic init");
     for (int it = 0; it < std::max(pc.maxIter, pc.minIter); ++it)
     {
-        dicApply(c, m, A, rD.p, r.p, w.p, stop);
+        dicApply(c, m, A, factor, rD.p, r.p, w.p, stop);
         launchDot(c, n, w.p, r.p, S + D_T0, 0);
         dicRhoK<<<1, 1, 0, c.stream>>>(S, F);
         dicDirK<<<blocks(n), kTpb, 0, c.stream>>>(n, w.p, p.p, S, F);

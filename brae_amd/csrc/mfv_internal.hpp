@@ -296,11 +296,11 @@ void launchDicPrecondition(Ctx& c, Mesh& m, const LduView& A, const double* r, d
 // bPrime (n, may be null): symGaussSeidel, each sweep followed by the reverse walk from the forward walk's bPrime
 void launchGaussSeidel(Ctx& c, Mesh& m, const LduView& A, const double* b, double* psi, int nSweeps,
                        double* bPrime = nullptr);
-// DIC's reciprocal diagonal (calcReciprocalD)
-void launchDicFactor(Ctx& c, Mesh& m, const LduView& A, double* rD);
+// DIC's reciprocal diagonal (calcReciprocalD); returns the factorisation (sweep.hpp), for the smoother
+unsigned launchDicFactor(Ctx& c, Mesh& m, const LduView& A, double* rD);
 // DICSmoother::smooth (gamg_solver_cpp.cu:277-293): per sweep psi += DIC(b - A psi); rA, w: n scratch each
-void launchDicSmooth(Ctx& c, Mesh& m, const LduView& A, const double* rD, const double* b, double* psi, int nSweeps,
-                     double* rA, double* w);
+void launchDicSmooth(Ctx& c, Mesh& m, const LduView& A, unsigned factor, const double* rD, const double* b, double* psi,
+                     int nSweeps, double* rA, double* w);
 // guarded: OpenFOAM GAMG's coarsest-level PCG-DIC (gamg_solver_cpp.cu:321-383): stop without an update
 // when |p.Ap|/normFactor < VSMALL, relTol counted only above 1e-20, no minIter
 PcgPerf pcgDicSolve(Ctx& c, Mesh& m, const LduView& A, const double* b, double* psi, const double* normFactor,

@@ -424,6 +424,7 @@ struct Level
     Mesh* m;
     LduView A;
     double* rD;
+    unsigned factor = 0;   // DIC's factorisation on its mesh
 };
 
 class Cycle
@@ -442,7 +443,7 @@ public:
                             w_.rD[gi].p};
         }
         if (dic())
-            for (Level& L : lv_) launchDicFactor(c_, *L.m, L.A, L.rD);
+            for (Level& L : lv_) L.factor = launchDicFactor(c_, *L.m, L.A, L.rD);
     }
 
     // GAMGSolver::Vcycle (gamg_solver_cpp.cu:627-735), on psi with its source; Apsi, fCorr scratch,
@@ -542,7 +543,7 @@ private:
     void smooth(Level& L, double* psi, const double* source, int nSweeps)
     {
         if (nSweeps <= 0) return;
-        if (dic()) launchDicSmooth(c_, *L.m, L.A, L.rD, source, psi, nSweeps, w_.tR.p, w_.tW.p);
+        if (dic()) launchDicSmooth(c_, *L.m, L.A, L.factor, L.rD, source, psi, nSweeps, w_.tR.p, w_.tW.p);
         if (g_.smoother == OfSmoother::GaussSeidel || g_.smoother == OfSmoother::DICGaussSeidel)
             launchGaussSeidel(c_, *L.m, L.A, source, psi, nSweeps);
         if (g_.smoother == OfSmoother::SymGaussSeidel) launchGaussSeidel(c_, *L.m, L.A, source, psi, nSweeps, w_.bPrime.p);

@@ -429,6 +429,7 @@ struct BicgRun
     LduView A;   // the folded matrix: diag is w.diagC
     int n;
     int gR;
+    SweepFactor dilu = 0;   // its factorisation, when factored in one launch
 
     // out = a.b (or the two sums t.s, t.t into out, out2), stop-aware
     void dot(const double* a, const double* b, double* out, int slot)
@@ -486,7 +487,7 @@ struct BicgRun
             diagApplyK<<<blocks(n), kTpb, 0, c.stream>>>(n, w.rD, r, y, w.fl);
             return;
         }
-        if (sweepSubstitute(c, m, w.rD, A.upper, A.lower, r, y, w.fl + BF_STOP)) return;
+        if (sweepSubstitute(c, m, dilu, w.rD, A.upper, A.lower, r, y, w.fl + BF_STOP)) return;
         const LevelSched& s = *m.sched;
         for (size_t l = 0; l + 1 < s.fwdStart.size(); ++l)
         {
@@ -508,7 +509,8 @@ struct BicgRun
             diagInvK<<<blocks(n), kTpb, 0, c.stream>>>(n, w.diagC, w.rD);
             return;
         }
-        if (sweepFactor(c, m, w.diagC, A.upper, A.lower, w.rD)) return;
+        dilu = sweepFactor(c, m, w.diagC, A.upper, A.lower, w.rD);
+        if (dilu) return;
         const LevelSched& s = *m.sched;
         for (size_t l = 0; l + 1 < s.fwdStart.size(); ++l)
         {

@@ -44,7 +44,8 @@ struct SweepPlan
     bool usable = false;      // false: the mesh keeps a launch per level
     bool lds = false;
     bool wide = false;        // a cell with more lower or owned faces than the narrow kernels load ahead
-    bool packed = false;      // LDS: the substitution's coefficients are the last factorisation's
+    SweepFactor factors = 0;  // the last factorisation
+    SweepFactor packed = 0;   // LDS: the one whose products are in aFwd, aBwd and dFwd (0: none)
     int n = 0, threads = 64;
     DBuf<int4> steps, gsSteps;     // the walks' steps
     DBuf<uint8_t> mem, gsMem;      // and the rest of them
@@ -971,8 +972,9 @@ template <int W>
 bool factorLds(Ctx& c, SweepPlan& p, const double* diag, const double* upper, const double* lower, double* rD)
 {
     const size_t bytes = ldsBytes(p);
-    p.packed = ldsAllowed(&ldsFactorK<W>, bytes) && ldsAllowed(&ldsSubstK<W>, bytes);
-    if (!p.packed) return false;
+    p.packed = 0;
+    if (!ldsAllowed(&ldsFactorK<W>, bytes) || !ldsAllowed(&ldsSubstK<W>, bytes)) return false;
+    p.packed = p.factors;
     const int nF = p.fwd.nEntries, nB = p.bwd.nEntries;
     packFactorK<<<blocks(std::max(nF, p.n)), kTpb, 0, c.stream>>>(nF, p.fwd.face, p.n, p.fwd.cell, diag, upper, lower,
                                                                  p.aFwd, p.dFwd);
@@ -983,12 +985,10 @@ bool factorLds(Ctx& c, SweepPlan& p, const double* diag, const double* upper, co
 }
 
 template <int W>
-bool substLds(Ctx& c, SweepPlan& p, const double* r, double* y, const int* stop)
+void substLds(Ctx& c, SweepPlan& p, const double* r, double* y, const int* stop)
 {
-    if (!p.packed) return false;
     ldsSubstK<W><<<1, p.threads, ldsBytes(p), c.stream>>>(p.n, ldsView(p.fwd, p.aFwd), ldsView(p.bwd, p.aBwd), p.dFwd,
                                                          r, y, stop);
-    return true;
 }
 
 template <int W, bool Factor>
@@ -1041,10 +1041,11 @@ void sweepPlan(Ctx& c, Mesh& m)
         m.sweep.reset(new SweepPlan());
 }
 
-bool sweepFactor(Ctx& c, Mesh& m, const double* diag, const double* upper, const double* lower, double* rD)
+SweepFactor sweepFactor(Ctx& c, Mesh& m, const double* diag, const double* upper, const double* lower, double* rD)
 {
     SweepPlan* p = planOf(m);
-    if (!p) return false;
+    if (!p) return 0;
+    if (++p->factors == 0) ++p->factors;
     bool done = true;
     if (p->lds)
         done = p->wide ? factorLds<kWide>(c, *p, diag, upper, lower, rD) : factorLds<kLdsNarrow>(c, *p, diag, upper, lower, rD);
@@ -1053,23 +1054,27 @@ bool sweepFactor(Ctx& c, Mesh& m, const double* diag, const double* upper, const
     else
         substFlow<kFlowNarrow, true>(c, *p, diag, upper, lower, nullptr, nullptr, rD, nullptr);
     hipCheck(hipGetLastError(), "sweep factor");
-    return done;
+    return done ? p->factors : 0;
 }
 
-bool sweepSubstitute(Ctx& c, Mesh& m, const double* rD, const double* upper, const double* lower, const double* r,
-                     double* y, const int* stop)
+bool sweepSubstitute(Ctx& c, Mesh& m, SweepFactor factor, const double* rD, const double* upper, const double* lower,
+                     const double* r, double* y, const int* stop)
 {
     SweepPlan* p = planOf(m);
-    if (!p) return false;
-    bool done = true;
+    if (!p || (p->lds && (factor == 0 || factor != p->packed))) return false;
     if (p->lds)
-        done = p->wide ? substLds<kWide>(c, *p, r, y, stop) : substLds<kLdsNarrow>(c, *p, r, y, stop);
+    {
+        if (p->wide)
+            substLds<kWide>(c, *p, r, y, stop);
+        else
+            substLds<kLdsNarrow>(c, *p, r, y, stop);
+    }
     else if (p->wide)
         substFlow<kWide, false>(c, *p, nullptr, upper, lower, rD, r, y, stop);
     else
         substFlow<kFlowNarrow, false>(c, *p, nullptr, upper, lower, rD, r, y, stop);
     hipCheck(hipGetLastError(), "sweep substitution");
-    return done;
+    return true;
 }
 
 bool sweepGaussSeidel(Ctx& c, Mesh& m, const double* diag, const double* upper, const double* b, double* psi,
