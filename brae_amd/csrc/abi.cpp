@@ -685,6 +685,15 @@ int mfv_amg_coarse_mode(mfv_amg amg, int mode, int* tailStart, int* ldsGrid, int
     return MFV_OK;
 }
 
+int mfv_amg_coarse_default(mfv_amg amg, int restore, int* inUse, int* firstGrid)
+{
+    if (!amg) return MFV_ERR_INVALID;
+    if (restore) amg->a.coarseMode = kCoarseDefault;
+    if (inUse) *inUse = amg->a.coarseMode == kCoarseDefault ? 1 : 0;
+    if (firstGrid) *firstGrid = amg->a.flowStart;
+    return MFV_OK;
+}
+
 int mfv_amg_fine_stencil(mfv_amg amg, int* nOffsets, int* hOffsets)
 {
     if (!amg || amg->a.grids.empty() || !nOffsets) return MFV_ERR_INVALID;

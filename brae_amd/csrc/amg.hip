@@ -25,7 +25,6 @@ namespace mfv {
 namespace {
 
 constexpr int kTpb = 256;
-constexpr int kMaxDenseCoarsest = 1024;   // the dense inverse's column buffer in LDS
 constexpr int kAlphaInBlockParts = 1024;  // corrAmulK partials a corrSmoothK workgroup reduces itself
 inline int blocks(long long n) { return (int)((n + kTpb - 1) / kTpb); }
 
@@ -1894,7 +1893,7 @@ Ts* vcycleAt(Ctx& c, Amg& a, int gi, const VcycleControls& vc, const int* stop,
         coarseApplyK<Tv, Ts><<<1, kTpb, 0, c.stream>>>(n, a.coarseInv.p, v.b, v.x, v.xm, up, stop);
         return v.x;
     }
-    if (gi == a.flowStart && !c.sequentialReduce && a.coarseMode == 3)
+    if (gi == a.flowStart && !c.sequentialReduce && a.coarseMode == kCoarseDefault)
     {
         ProfScope ps(c, kProfGridDown + gi);
         if (vc.nPre == 0) zeroK<Ts><<<blocks(n), kTpb, 0, c.stream>>>(n, v.x, stop);

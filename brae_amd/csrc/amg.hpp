@@ -126,6 +126,12 @@ struct OfWork
     DBuf<double> dense;                             // gamg.cu's coarsest elimination: n*n matrix + n rhs
 };
 
+// the most cells a coarsest grid may have: the dense inverse's column buffer in LDS
+constexpr int kMaxDenseCoarsest = 1024;
+
+// the coarse mode while none is set: the small grids in one launch of many workgroups (cycle_flow.hip)
+constexpr int kCoarseDefault = 3;
+
 struct Amg
 {
     int nFine = 0;
@@ -145,9 +151,8 @@ struct Amg
     int tailStart = 0;             // first grid the single-workgroup tail kernel runs (0: none)
     DBuf<uint8_t> tailDesc;        // per tail grid: pointers and sizes for the tail kernel
     int tailFor = -1;              // precision the descriptors were built for (-1: stale)
-    int coarseMode = 3;            // 0: per-grid kernels; 1: the one-workgroup tail; 2: that tail with its
-                                   // coarsest grids staged in LDS, as many as fit (else 1); 3 (until a mode is
-                                   // set): the small grids in one launch of many waves (cycle_flow.hip)
+    int coarseMode = kCoarseDefault;   // 0: per-grid kernels; 1: the one-workgroup tail; 2: that tail with its
+                                       // coarsest grids staged in LDS, as many as fit (else 1)
     DBuf<uint8_t> tailLdsBlob;     // the LDS-staged tail's slice starts, 16-bit columns and lists
     DBuf<uint8_t> tailLdsDesc;     // its descriptor
     int tailLdsBytes = 0;          // LDS it needs (0: the tail does not fit; tailK runs)

@@ -46,7 +46,6 @@ constexpr int kFlowRows = 1 << 13;
 // 64, 128 and 256 workgroups: 66, 55 and 48 us at 7,793 rows, but 105, 94 and 96 at 4,584 with the scaled correction
 // and 6.2 against 6.3 ms for the solve over 45 k cells with 128 and 256
 constexpr int kFlowGroups = 128;
-constexpr int kMaxCoarsest = 1024;
 constexpr int kStagedCoarsest = 64;   // the coarsest inverse's rows go through LDS up to this size
 
 // a vector entry as its stored form reads back (FP16: rounded under the multiplier m, saturated)
@@ -327,7 +326,7 @@ __global__ __launch_bounds__(kThreads) void flowCycleK(const FlowGrid* __restric
                                                  const int* __restrict__ stop)
 {
     if (stop && *stop) return;
-    __shared__ double sb[kMaxCoarsest];
+    __shared__ double sb[kMaxDenseCoarsest];
     __shared__ double sInv[64 * (kStagedCoarsest + 1)];
     __shared__ int slots[2];
     __shared__ int chunksOf[kMaxFlowGrids];
@@ -627,14 +626,14 @@ __global__ __launch_bounds__(kThreads) void zeroWordsK(size_t n, Word* __restric
 // The launch's arrays for a.prec: descriptors, columns (a patterned grid's written out) and their coarse cells,
 // and the words. They are written on the device: by the host they made a new hierarchy's first FP64 set-up 1.6 ms at
 // 45 k cells and 1.5 at 8,000; so it is 1.2 and 1.0 (before this launch and the staged inverse 1.2 and 1.3).
-// a.flowStart: the first grid of at most kFlowRows rows, or -1 where none has a coarser one.
+// a.flowStart: the first grid of at most kFlowRows rows, or -1 where none has a coarser one (or over kMaxFlowGrids do).
 void flowCycleBuild(Ctx& c, Amg& a)
 {
     const int nG = (int)a.grids.size();
     a.flowStart = -1;
     for (int g = 0; g + 1 < nG && a.flowStart < 0; ++g)
         if (a.grids[g].n <= kFlowRows) a.flowStart = g;
-    if (a.flowStart < 0 || nG - a.flowStart > kMaxFlowGrids || a.grids.back().n > kMaxCoarsest)
+    if (a.flowStart < 0 || nG - a.flowStart > kMaxFlowGrids)
     {
         a.flowStart = -1;
         return;

@@ -187,6 +187,7 @@ _SIGS = {
     "mfv_amg_grid_size": [P, I, P, P],
     "mfv_amg_fine_stencil": [P, P, P],
     "mfv_amg_coarse_mode": [P, I, P, P, P],
+    "mfv_amg_coarse_default": [P, I, P, P],
     "mfv_amg_pcg_solve_batch": [P, I, P, P],
     "mfv_fold_boundary_diag": [P, P, P, P, P, P, P],
     "mfv_reciprocal_v": [P, P, P, P, P],
@@ -520,12 +521,21 @@ class Amg:
 
     def coarse_mode(self, mode=-1):
         """sets how the coarsest grids run (0 per-grid kernels, 1 one workgroup, 2 one workgroup with the
-        coarsest grids staged in LDS; -1 leaves it; until a mode is set, one launch of many workgroups) and returns (the tail's first grid, the first grid
-        staged, the LDS bytes the staged grids take)"""
+        coarsest grids staged in LDS; -1 leaves it; coarse_default() returns to the default, one launch of many
+        workgroups) and returns what the one workgroup's tail is: (its first grid, the first grid staged, the
+        LDS bytes the staged grids take)"""
         t, g, b = ctypes.c_int(), ctypes.c_int(), ctypes.c_int()
         self.ctx._check(lib().mfv_amg_coarse_mode(self.h, mode, ctypes.byref(t), ctypes.byref(g), ctypes.byref(b)),
                         "amg_coarse_mode")
         return t.value, g.value, b.value
+
+    def coarse_default(self, restore=True):
+        """returns to the default way of running the coarsest grids (restore=False: only asks) and returns
+        (whether it is in use, its one launch's first grid or -1 where the hierarchy has none)"""
+        u, g = ctypes.c_int(), ctypes.c_int()
+        self.ctx._check(lib().mfv_amg_coarse_default(self.h, int(restore), ctypes.byref(u), ctypes.byref(g)),
+                        "amg_coarse_default")
+        return bool(u.value), g.value
 
     def level(self, i):
         import numpy as np

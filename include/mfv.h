@@ -342,16 +342,22 @@ int mfv_amg_grid_size(mfv_amg amg, int grid, int* nCells, int* nFaces);
  * offsets. 0 offsets: the fine matrix is read as sliced rows. */
 int mfv_amg_fine_stencil(mfv_amg amg, int* nOffsets, int* hOffsets);
 /* How the coarsest grids' cycle runs, no counterpart in the reference (its small levels run one kernel
- * per step). Until a mode is set, the grids from the first one of at most 8192 cells down run in one
- * launch of many workgroups that hand the steps' values on to each other. The modes below 4096 cells
- * run the grids from the first such one down in one workgroup (the tail): mode 2 stages the tail's
- * coarsest grids -- as many as fit the device's LDS per workgroup -- in that workgroup's LDS and reads
- * the others where they are; mode 1 reads them all where they are; mode 0 runs every grid with its own
- * kernels. All give the same bits, except that the scaled correction keeps mode 1's kernel in mode 2
- * and takes its sums in another order until a mode is set. mode -1 only queries. *tailStart: the tail's first grid (0: no tail);
- * *ldsGrid: the first grid staged (0: none); *ldsBytes: the LDS the staged grids take, in the precision
- * of the last mfv_amg_galerkin; any of the three may be NULL. */
+ * per step). By default the grids from the first one of at most 8192 cells down run in one launch of many
+ * workgroups that hand the steps' values on to each other. The modes replace that, until
+ * mfv_amg_coarse_default: modes 1 and 2 run the grids from the first one of at most 4096 cells down in one
+ * workgroup (the tail), mode 2 with the tail's coarsest grids -- as many as fit the device's LDS per
+ * workgroup -- staged in that workgroup's LDS and the others read where they are, mode 1 with all of them
+ * read where they are; mode 0 runs every grid with its own kernels. All give the same bits, except that the
+ * scaled correction keeps mode 1's kernel in mode 2 and takes its sums in another order by default. mode -1
+ * only queries what the tail of modes 1 and 2 is, whether it is in use or not. *tailStart: the tail's first
+ * grid (0: no tail); *ldsGrid: the first grid staged (0: none); *ldsBytes: the LDS the staged grids take, in
+ * the precision of the last mfv_amg_galerkin; any of the three may be NULL. */
 int mfv_amg_coarse_mode(mfv_amg amg, int mode, int* tailStart, int* ldsGrid, int* ldsBytes);
+/* With restore != 0, back to the default after mfv_amg_coarse_mode. *inUse: 1 while no mode is set;
+ * *firstGrid: the first grid of the default's one launch in the precision of the last mfv_amg_galerkin, or
+ * -1 where the hierarchy has none (no grid of at most 8192 cells has a coarser one; its grids then run as in
+ * mode 2). Sequential reductions use the per-grid kernels in any mode. Either may be NULL. */
+int mfv_amg_coarse_default(mfv_amg amg, int restore, int* inUse, int* firstGrid);
 /* host copies of the step from grid `level` to grid `level+1` (any pointer may be NULL):
  * restrict map [nCells(level)], coarse owner/neighbour [nFaces(level+1)], faceRestrict and faceFlip
  * [nFaces(level)] -- AMGLevel's map/cOwn/cNei/faceRestrict/faceFlip (device_amg.cuh:119-182) */
