@@ -330,6 +330,7 @@ __global__ __launch_bounds__(kThreads) void flowCycleK(const FlowGrid* __restric
     __shared__ double sInv[64 * (kStagedCoarsest + 1)];
     __shared__ int slots[2];
     __shared__ int chunksOf[kMaxFlowGrids];
+    __shared__ double sums[2 * (kThreads / 64)];
     const int lane = threadIdx.x & 63, quarter = (int)__builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const unsigned tag = launchTag(state);
     GroupChunks order(state, slots);
@@ -536,13 +537,18 @@ __global__ __launch_bounds__(kThreads) void flowCycleK(const FlowGrid* __restric
                     den = (double)ec * (double)ae;
                 }
             }
+            // the chunk's sums, its waves' in order
             num = waveSum(num);
             den = waveSum(den);
             if (lane == 0)
             {
-                Hand<double>::put(G.sums, 2 * part, tag, num);
-                Hand<double>::put(G.sums, 2 * part + 1, tag, den);
+                sums[2 * quarter] = num;
+                sums[2 * quarter + 1] = den;
             }
+            __syncthreads();
+            if (threadIdx.x < 2)
+                Hand<double>::put(G.sums, 2 * (t - first) + (int)threadIdx.x, tag,
+                                  ((sums[threadIdx.x] + sums[threadIdx.x + 2]) + sums[threadIdx.x + 4]) + sums[threadIdx.x + 6]);
         }
         else   // kScaleUpdate
         {
@@ -558,8 +564,10 @@ __global__ __launch_bounds__(kThreads) void flowCycleK(const FlowGrid* __restric
                 oa.ask(G.ae, c, tag);
                 oe.ask(grids[g + 1].f, mc, tag);
             }
+            // the grid's sums over its chunks, taken by the workgroup: were every wave to ask for a pair of every wave's,
+            // as many words would cross as the grid has rows, squared
             double num = 0.0, den = 0.0;
-            for (int q = lane; q < 4 * chunks; q += 64)
+            for (int q = threadIdx.x; q < chunks; q += kThreads)
             {
                 const int i[2] = {2 * q, 2 * q + 1};
                 double v[2];
@@ -569,6 +577,14 @@ __global__ __launch_bounds__(kThreads) void flowCycleK(const FlowGrid* __restric
             }
             num = waveSum(num);
             den = waveSum(den);
+            if (lane == 0)
+            {
+                sums[2 * quarter] = num;
+                sums[2 * quarter + 1] = den;
+            }
+            __syncthreads();
+            num = ((sums[0] + sums[2]) + sums[4]) + sums[6];
+            den = ((sums[1] + sums[3]) + sums[5]) + sums[7];
             const Tv al = (Tv)(den > 1e-30 ? num / den : 1.0);
             if (on)
             {
@@ -645,7 +661,7 @@ void flowCycleBuild(Ctx& c, Amg& a)
     {
         const Grid& G = a.grids[a.flowStart + t];
         entryAt[t + 1] = entryAt[t] + (t + 1 < T ? (size_t)G.sell.nnz : 0);
-        wordAt[t + 1] = wordAt[t] + 8 * per * (size_t)G.n + 16 * (((size_t)G.n + 63) / 64);
+        wordAt[t + 1] = wordAt[t] + 8 * per * (size_t)G.n + 4 * (((size_t)G.n + 63) / 64);
     }
     // the columns depend on the structure alone
     if (a.flowCols.n != 2 * entryAt[T])
@@ -698,7 +714,7 @@ void flowCycleBuild(Ctx& c, Amg& a)
         q.y[1] = take(rows);
         q.f = take(rows);
         q.ae = take(rows);
-        q.sums = take(16 * (((size_t)G.n + 63) / 64));
+        q.sums = take(4 * (((size_t)G.n + 63) / 64));
     }
     a.flowDesc.upload(reinterpret_cast<const uint8_t*>(d.data()), d.size() * sizeof(FlowGrid), c.stream);
 }
