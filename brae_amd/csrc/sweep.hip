@@ -467,7 +467,27 @@ __device__ __forceinline__ void laneLoad(const int4* __restrict__ steps, int s, 
     }
 }
 
-// The values of a lane's first W entries; need: a bit per entry. Each poll reads all of them unconditionally
+// The entries from k0 on (those past the step's marked missing). A chunk with wide rows takes its entries W at a time:
+// one after the other each cost the loads of its face and place, of its coefficient and of its value in a chain (110
+// levels of 2,700 cells with up to 25 lower faces: 52 us a level, 22 so, 31 with a launch per level).
+template <int W>
+__device__ __forceinline__ void laneMore(int k0, const int* __restrict__ face, const int* __restrict__ pos, const int4 d,
+                                         int (&f)[W], int (&p)[W])
+{
+    const int j = min((int)threadIdx.x, d.y - 1);
+#pragma unroll
+    for (int k = 0; k < W; ++k)
+    {
+        const int e = d.z + min(k0 + k, d.w - 1) * d.y + j;
+        f[k] = face[e];
+        p[k] = pos[e];
+    }
+#pragma unroll
+    for (int k = 0; k < W; ++k)
+        if (k0 + k >= d.w) f[k] = -1;
+}
+
+// The values of a lane's W entries; need: a bit per entry. Each poll reads all of them unconditionally
 // (an entry that is not needed names a place in bounds), so it costs one round trip, not one per entry.
 template <int W>
 __device__ __forceinline__ void awaitAll(const Word* hand, const int (&pos)[W], unsigned need,
@@ -509,31 +529,27 @@ __global__ __launch_bounds__(64) void flowSubstK(PlanView P, const double* __res
             const int own = L.self;
             const double rd = Factor ? 0.0 : rD[L.c];
             const double v0 = back ? 0.0 : (Factor ? diag[L.c] : r[L.c]);
-            double a[W], x[W];
-            unsigned need = 0;
-#pragma unroll
-            for (int k = 0; k < W; ++k)
-            {
-                const int f = max(L.face[k], 0);
-                a[k] = Factor ? upper[f] * lower[f] : rd * (back ? upper[f] : lower[f]);
-                need |= (L.face[k] >= 0 ? 1u : 0u) << k;
-            }
             const unsigned want = back ? tag + 1 : tag;
-            const unsigned has = need;
-            double v = back ? awaitValue<double>(hand, own, tag) : (Factor ? v0 : rd * v0);   // there long before the neighbours'
-            awaitAll<W>(hand, L.pos, need, want, x);
-#pragma unroll
-            for (int k = 0; k < W; ++k)
-                if (has >> k & 1u) v = Factor ? v - a[k] / x[k] : v - a[k] * x[k];
-            for (int k = W; k < L.d.w; ++k)
+            double v = 0.0;
+            for (int k0 = 0; k0 < L.d.w; k0 += W)
             {
-                const int e = L.d.z + k * L.d.y + lane, f = P.face[back][e];
-                if (f < 0) break;
-                const double xk = awaitValue<double>(hand, P.pos[back][e], want);
-                if (Factor)
-                    v -= upper[f] * lower[f] / xk;
-                else
-                    v -= rd * (back ? upper[f] : lower[f]) * xk;
+                if (k0) laneMore<W>(k0, P.face[back], P.pos[back], L.d, L.face, L.pos);
+                double a[W], x[W];
+                unsigned need = 0;
+#pragma unroll
+                for (int k = 0; k < W; ++k)
+                {
+                    const int f = max(L.face[k], 0);
+                    a[k] = Factor ? upper[f] * lower[f] : rd * (back ? upper[f] : lower[f]);
+                    need |= (L.face[k] >= 0 ? 1u : 0u) << k;
+                }
+                const unsigned has = need;
+                if (!k0)   // its own is there long before the neighbours'
+                    v = back ? awaitValue<double>(hand, own, tag) : (Factor ? v0 : rd * v0);
+                awaitAll<W>(hand, L.pos, need, want, x);
+#pragma unroll
+                for (int k = 0; k < W; ++k)
+                    if (has >> k & 1u) v = Factor ? v - a[k] / x[k] : v - a[k] * x[k];
             }
             Hand<double>::put(hand, own, want, v);
             if (Factor)
@@ -567,45 +583,31 @@ __global__ __launch_bounds__(64) void flowGsK(int nSteps, const int4* __restrict
             const int nl = Back ? L.d.w : L.self;   // the entries handed over: all, or the lower ones
             double v = Back ? bPrime[L.c] : b[L.c];
             const double dg = diag[L.c];
-            double a[W], x[W];
-            unsigned has = 0, need = 0;
-#pragma unroll
-            for (int k = 0; k < W; ++k)
+            if (!Back && bPrime && nl == 0) bPrime[L.c] = v;
+            // the reverse walk from its last entries
+            const int last = Back ? (L.d.w - 1) / W * W : 0;
+            for (int k0 = last; Back ? k0 >= 0 : k0 < L.d.w; k0 += Back ? -W : W)
             {
-                a[k] = upper[max(L.face[k], 0)];
-                const bool on = L.face[k] >= 0;
-                has |= (on ? 1u : 0u) << k;
-                need |= (on && k < nl ? 1u : 0u) << k;
-                if (on && k >= nl) x[k] = psi[L.pos[k]];
-            }
-            awaitAll<W>(hand, L.pos, need, tag, x);
-            if (Back)
-            {
-                for (int k = L.d.w - 1; k >= W; --k)
-                {
-                    const int e = L.d.z + k * L.d.y + lane, f = face[e];
-                    if (f >= 0) v -= upper[f] * awaitValue<double>(hand, pos[e], tag);
-                }
-#pragma unroll
-                for (int k = W - 1; k >= 0; --k)
-                    if (has >> k & 1u) v -= a[k] * x[k];
-            }
-            else
-            {
-                if (bPrime && nl == 0) bPrime[L.c] = v;
+                if (Back ? last > 0 : k0 > 0) laneMore<W>(k0, face, pos, L.d, L.face, L.pos);
+                double a[W], x[W];
+                unsigned has = 0, need = 0;
 #pragma unroll
                 for (int k = 0; k < W; ++k)
-                    if (has >> k & 1u)
-                    {
-                        v -= a[k] * x[k];
-                        if (bPrime && k + 1 == nl) bPrime[L.c] = v;
-                    }
-                for (int k = W; k < L.d.w; ++k)
                 {
-                    const int e = L.d.z + k * L.d.y + lane, f = face[e];
-                    if (f < 0) break;
-                    v -= upper[f] * (k < nl ? awaitValue<double>(hand, pos[e], tag) : psi[pos[e]]);
-                    if (bPrime && k + 1 == nl) bPrime[L.c] = v;
+                    a[k] = upper[max(L.face[k], 0)];
+                    const bool on = L.face[k] >= 0;
+                    has |= (on ? 1u : 0u) << k;
+                    need |= (on && k0 + k < nl ? 1u : 0u) << k;
+                    if (on && k0 + k >= nl) x[k] = psi[L.pos[k]];
+                }
+                awaitAll<W>(hand, L.pos, need, tag, x);
+#pragma unroll
+                for (int j = 0; j < W; ++j)
+                {
+                    const int k = Back ? W - 1 - j : j;
+                    if (!(has >> k & 1u)) continue;
+                    v -= a[k] * x[k];
+                    if (!Back && bPrime && k0 + k + 1 == nl) bPrime[L.c] = v;
                 }
             }
             v /= dg;
