@@ -74,6 +74,12 @@ constexpr int kLdsThreads = 512;
 // 3.3x at 200^3, 2.0x at 272^3 (20 M cells, 165 -> 83 ms); the plan takes about 76 bytes a cell of a hex mesh, and
 // 52 more with Gauss-Seidel's walk.
 constexpr int kFlowMaxCells = 1 << 25;
+// A mesh of so few levels keeps a launch per level too: its sweep is a stream over the cells, which a launch a level
+// runs with the whole chip, one workgroup or kFlowWaves waves with a part of it. A DIC application, one launch a sweep
+// and a launch per level, us: cells in two colours (two levels) 51 and 36 on 16^3 cells, 131 and 38 on 27^3, 213 and
+// 110 on 64^3, 636 and 153 on 1 M; numbered at random (16 to 20 levels) 75 and 205, 159 and 316, 236 and 512, 697 and
+// 802; at 4.1 M 2,640 and 2,400, two Gauss-Seidel sweeps 2,100 and 2,660.
+int fewLevels(int n, bool lds) { return lds ? 3 + n / 3200 : 2 + std::min(10, n / 60000); }
 // Entries of a step's cell that are loaded ahead, by the most that a cell of the mesh has (a hex mesh's have
 // three lower and three owned faces, agglomerated ones more); a cell's entries past these are loaded where
 // they are used. Substitution in LDS (in pairs) and by flow, Gauss-Seidel in LDS and by flow:
@@ -890,7 +896,7 @@ bool planBuild(Ctx& c, Mesh& m, SweepPlan* p)
     return true;
 }
 
-// the mesh's plan, or null: a mesh without faces or above kFlowMaxCells, or a plan that would not fit
+// the mesh's plan, or null: a mesh without faces, above kFlowMaxCells or of few levels, or a plan that would not fit
 SweepPlan* planOf(const Mesh& m) { return m.sweep && m.sweep->usable ? m.sweep.get() : nullptr; }
 
 // the forward walk of Gauss-Seidel (both runs of a cell's faces), on the first such sweep outside a capture
@@ -1036,7 +1042,8 @@ void gsFlow(Ctx& c, SweepPlan& p, const Walk& w, const double* diag, const doubl
 void sweepPlan(Ctx& c, Mesh& m)
 {
     m.sweep.reset(new SweepPlan());
-    if (!m.nFaces || m.nCells > kFlowMaxCells) return;
+    const size_t levels = std::max(m.sched->fwdStart.size(), m.sched->bwdStart.size()) - 1;
+    if (!m.nFaces || m.nCells > kFlowMaxCells || (int)levels <= fewLevels(m.nCells, m.nCells <= kLdsCells)) return;
     if (fits([&] { return planBuild(c, m, m.sweep.get()); }))
         m.sweep->usable = true;
     else

@@ -1,7 +1,7 @@
 // The sequential sweeps in one launch each (sweep.hip): DIC's and DILU's factorisation, their forward and
 // backward substitution, and Gauss-Seidel, on a plan built with the mesh's level schedule. Each sweep returns
-// false, having done nothing, where it belongs to the caller's launch-per-level path: a mesh above kFlowMaxCells,
-// a plan that does not fit, or a first Gauss-Seidel inside a capture (its walk is laid out by the first one).
+// false, having done nothing, where it belongs to the caller's launch-per-level path: a mesh above kFlowMaxCells or
+// of few levels, a plan that does not fit, or a first Gauss-Seidel inside a capture (its walk is laid out by the first one).
 #pragma once
 
 #include "mfv_internal.hpp"

@@ -1,6 +1,6 @@
 """Sweeps in one launch on meshes unlike a box in its natural order: rows of many faces above the LDS size, and cells
-in a few wide levels (colours). Results to the bit against the oracle, and wide rows not left far slower than the chain of
-levels they are."""
+in a few wide levels (colours). Results to the bit against the oracle, and no shape left far slower than the work it
+is: a chain of levels in the first case, a stream over the cells in the second."""
 import ctypes
 import time
 
@@ -93,6 +93,14 @@ def test_bits(name):
     for symmetric in (False, True):
         assert np.array_equal(S.gauss_seidel(symmetric),
                               O.gauss_seidel(S.n, S.own, S.nei, S.diag, S.up, S.b, S.x0, 2, symmetric=symmetric)), symmetric
+
+
+def test_two_colours_are_a_stream():
+    """1 M cells in 2 levels against the same box in its natural order, 318 levels: 0.15 of its time with a launch per
+    level, 0.63 when the waves of the one launch took their chunks one after another"""
+    t = [Sweeps(m).dic_seconds() for m in (coloured(128, 128, 64, 2), box(128, 128, 64))]
+    print("case: two colours", t, flush=True)
+    assert t[0] < 0.35 * t[1]
 
 
 def test_wide_rows_are_loaded_together():
