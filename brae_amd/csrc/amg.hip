@@ -1893,7 +1893,7 @@ Ts* vcycleAt(Ctx& c, Amg& a, int gi, const VcycleControls& vc, const int* stop,
         coarseApplyK<Tv, Ts><<<1, kTpb, 0, c.stream>>>(n, a.coarseInv.p, v.b, v.x, v.xm, up, stop);
         return v.x;
     }
-    if (gi == a.flowStart && !c.sequentialReduce && a.coarseMode == kCoarseDefault)
+    if (gi == a.flowStart && !c.sequentialReduce && a.coarseMode == kCoarseDefault && flowCycleRuns(a, vc))
     {
         ProfScope ps(c, kProfGridDown + gi);
         if (vc.nPre == 0) zeroK<Ts><<<blocks(n), kTpb, 0, c.stream>>>(n, v.x, stop);

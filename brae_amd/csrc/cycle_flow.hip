@@ -719,6 +719,17 @@ void flowCycleBuild(Ctx& c, Amg& a)
     a.flowDesc.upload(reinterpret_cast<const uint8_t*>(d.data()), d.size() * sizeof(FlowGrid), c.stream);
 }
 
+// A step here costs the time a value takes between two CUs, in one workgroup a barrier: on a few hundred rows the one
+// workgroup's many sweeps are the faster. V(4,3) on 512, 1,600 (2-D) and 1,728 (3-D) cells, here and there, us: FP64
+// 61 and 51, 87 and 73, 98 and 99; FP16 62 and 61, 90 and 75, 98 and 89. On 4,096 122 and 148, 119 and 120; V(2,1) on
+// 1,600 and 1,728 46 and 45, 52 and 59. The one workgroup's coarsest solve has to be small: 962 cells take it 250.
+bool flowCycleRuns(const Amg& a, const VcycleControls& vc)
+{
+    constexpr int kFewRows = 2048, kManySweeps = 5, kFewCoarsest = 128;
+    if (a.flowStart < 0) return false;
+    return vc.nPre + vc.nPost < kManySweeps || a.grids[a.flowStart].n > kFewRows || a.nCoarsest > kFewCoarsest;
+}
+
 template <typename Tm, typename Tv, typename Ts>
 void flowCycle(Ctx& c, Amg& a, const VcycleControls& vc, const Ts* b, const Ts* x, Ts* out, const Scatter<Tv, Ts>& up,
                const int* stop)

@@ -9,6 +9,9 @@ namespace mfv {
 // lays the launch's arrays out for the hierarchy's current precision (after its vectors are allocated)
 void flowCycleBuild(Ctx& c, Amg& a);
 
+// whether a cycle's small grids go through it (a.coarseMode aside)
+bool flowCycleRuns(const Amg& a, const VcycleControls& vc);
+
 // Runs the cycle from grid a.flowStart to the coarsest and back on that grid's b and x (0 without pre-sweeps). Its
 // values go to `up` and, unless null, to `out`, which is not x: rows read their neighbours' x until the end. Needs
 // a.flowStart >= 0.

@@ -356,7 +356,7 @@ int mfv_amg_coarse_mode(mfv_amg amg, int mode, int* tailStart, int* ldsGrid, int
 /* With restore != 0, back to the default after mfv_amg_coarse_mode. *inUse: 1 while no mode is set;
  * *firstGrid: the first grid of the default's one launch in the precision of the last mfv_amg_galerkin, or
  * -1 where the hierarchy has none (no grid of at most 8192 cells has a coarser one; its grids then run as in
- * mode 2). Sequential reductions use the per-grid kernels in any mode. Either may be NULL. */
+ * mode 2, as do those of cycles of five or more sweeps on at most 2048 cells). Sequential reductions use the per-grid kernels in any mode. Either may be NULL. */
 int mfv_amg_coarse_default(mfv_amg amg, int restore, int* inUse, int* firstGrid);
 /* host copies of the step from grid `level` to grid `level+1` (any pointer may be NULL):
  * restrict map [nCells(level)], coarse owner/neighbour [nFaces(level+1)], faceRestrict and faceFlip
