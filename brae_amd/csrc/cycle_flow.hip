@@ -44,7 +44,7 @@ constexpr int kMaxFlowGrids = 32;
 // ms against 6.2 (4,847 rows, FP64), 13.0 against 12.8 (7,793, FP16).
 constexpr int kFlowRows = 1 << 13;
 // 64, 128 and 256 workgroups: 66, 55 and 48 us at 7,793 rows, but 105, 94 and 96 at 4,584 with the scaled correction
-// and 6.2 against 6.3 ms for the solve over 45 k cells with 128 and 256
+// and 6.2 against 6.3 ms for the solve over 45 k cells with 128 and 256 (as first built; 128 now take 46 and 78)
 constexpr int kFlowGroups = 128;
 constexpr int kStagedCoarsest = 64;   // the coarsest inverse's rows go through LDS up to this size
 

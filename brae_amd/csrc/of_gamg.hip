@@ -560,7 +560,7 @@ private:
     }
 
     // On levels of a few hundred to a few thousand cells launches are the cost: the product and its two sums in one,
-    // the sums finished by the update's workgroups, so two launches where six were: a solve over 13,861 cells 42.5
+    // the sums finished by the update's workgroups, so two launches where six were: a solve over 12,180 cells 42.5
     // -> 40.8 ms (41.5 with the finishing launches kept). Above kScaleParts partials, which every workgroup would
     // read, two finishing launches come in between; at 65 k to 590 k cells neither way is the faster.
     void scale(Level& L, double* field, double* Acf, const double* source)

@@ -15,7 +15,7 @@
 // path's and the host's to the bit.
 // Measured, a launch per level before: one DILU application on 64^3 cells (forward and backward, 380 levels)
 // 1,280 -> 196 us, 0.5 us a level, the time a value takes between two CUs; OpenFOAM's GAMG with Gauss-Seidel
-// on a 2-D mesh of 12,180 cells 470 -> 70 ms, 42 with successive sweeps overlapped.
+// on a 2-D mesh of 12,180 cells 486 -> 62.6 ms, and 61 -> 42.7 with successive sweeps overlapped.
 #include "handover.hpp"
 #include "sweep.hpp"
 
@@ -294,7 +294,7 @@ __global__ __launch_bounds__(kLdsThreads) void ldsSubstK(int n, LdsWalk F, LdsWa
 // One sweep is bound by its chain of levels, 0.33 us each, with most of a workgroup's room unused. The
 // neighbours of a step lie at most lag - 1 steps from it, so sweep s + 1 may take a step once sweep s has taken
 // the lag - 1 steps after it: teams of `team` threads walk successive sweeps lag steps apart, in the same
-// barriers, and no step reads what another team writes between two of them: two sweeps over 13,861 cells in 250
+// barriers, and no step reads what another team writes between two of them: two sweeps over 12,180 cells in 250
 // levels 164 -> 104 us, four over their agglomerates 70 -> 42. Symmetric sweeps take turns (one team).
 template <int W, int WB, bool Sym>
 __global__ __launch_bounds__(kLdsThreads) void ldsGsK(int n, LdsWalk F, LdsWalk B, double* in, double* __restrict__ psi,
