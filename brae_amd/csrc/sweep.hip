@@ -78,8 +78,9 @@ constexpr int kFlowMaxCells = 1 << 25;
 // runs with the whole chip, one workgroup or kFlowWaves waves with a part of it. A DIC application, one launch a sweep
 // and a launch per level, us: cells in two colours (two levels) 51 and 36 on 16^3 cells, 131 and 38 on 27^3, 213 and
 // 110 on 64^3, 636 and 153 on 1 M; numbered at random (16 to 20 levels) 75 and 205, 159 and 316, 236 and 512, 697 and
-// 802; at 4.1 M 2,640 and 2,400, two Gauss-Seidel sweeps 2,100 and 2,660.
-int fewLevels(int n, bool lds) { return lds ? 3 + n / 3200 : 2 + std::min(10, n / 60000); }
+// 802; at 4.1 M 2,640 and 2,400, two Gauss-Seidel sweeps 2,100 and 2,660. On a few hundred cells, GAMG's coarse grids,
+// the launches are the cost whatever the levels: there only a mesh of one level has no plan.
+int fewLevels(int n, bool lds) { return lds ? std::min(9, 1 + n / 1700) : 2 + std::min(10, n / 60000); }
 // Entries of a step's cell that are loaded ahead, by the most that a cell of the mesh has (a hex mesh's have
 // three lower and three owned faces, agglomerated ones more); a cell's entries past these are loaded where
 // they are used. Substitution in LDS (in pairs) and by flow, Gauss-Seidel in LDS and by flow:
